@@ -107,6 +107,7 @@ struct kw_plan {
   bool tuned = false;
   bool col_wide = false;  // KW_COL_WIDE=1: no narrow-tile fallback on small grids
   int col_persist = 3;    // KW_COL_PERSIST: column passes that loop over tiles (ColArgs::persist)
+  int col_small = 1;      // small-grid column passes (ColArgs::small); KW_COL_SMALL=0/1/2
   int col_grid = 0;       // KW_COL_GRID: workgroups per instance of looping passes (0: resident grid)
   bool inst_dirty = true;
   // per-kernel timing (kw_plan_run_profiled)
@@ -212,6 +213,7 @@ int ypass(kw_plan* P, int mode, const std::vector<int>& bufs) {
   a.wide = P->col_wide;
   a.persist = P->col_persist;
   a.grid = P->col_grid;
+  a.small = P->col_small;
   a.nbuf = (int)bufs.size();
   for (size_t i = 0; i < bufs.size(); ++i) a.bufs[i] = bufs[i];
   const double spec_bytes = 8.0 * P->nb * (double)P->g.rows * P->g.nh;
@@ -226,6 +228,7 @@ int xpass(kw_plan* P, const std::vector<XJob>& jobs, int kind) {
   a.wide = P->col_wide;
   a.persist = P->col_persist;
   a.grid = P->col_grid;
+  a.small = P->col_small;
   a.njob = (int)jobs.size();
   int nin = 0, last = -1;
   for (size_t i = 0; i < jobs.size(); ++i) {
@@ -430,6 +433,10 @@ int kw_plan_create(const kw_plan_desc* d, kw_plan** out) {
     if (pe && pe[0] >= '0' && pe[0] <= '3') P->col_persist = pe[0] - '0';
     const char* ge = std::getenv("KW_COL_GRID");
     P->col_grid = ge ? std::max(0, std::atoi(ge)) : 0;
+    // a caller that forces tile widths, radix plans or looping grids gets the passes those switches are for
+    const char* sm = std::getenv("KW_COL_SMALL");
+    const bool forced = P->col_wide || P->col_grid > 0 || std::getenv("KW_COL_TILES") || std::getenv("KW_COL_PLANS");
+    P->col_small = sm && sm[0] >= '0' && sm[0] <= '2' ? sm[0] - '0' : forced ? 0 : 1;
   }
   int rc = KW_OK;
   auto cleanup = [&](int code) { delete P; return code; };

@@ -9,6 +9,15 @@ namespace kw {
 
 constexpr int kColDevices = 64;
 
+// Largest pass, in lanes over all its jobs or buffers, that takes the small-grid form
+// (k_col_small): about half the lanes the chip holds at these kernels' registers.  Below,
+// one pass is a chain of latencies (us per step before -> with the form: 128^2 50.9 ->
+// 39.8, 512^2 power law 86.7 -> 72.4, 64^3 power law 116.5 -> 91.2, 64 maps of 128^2 with
+// 133 k lanes a pass 75.8 -> 68.7); above, the narrow tiles' short memory runs cost more
+// than the chain (four 640^2 plus four 512 x 768 lines, 164 k and 197 k lanes a pass: 204
+// either way with the first in this form, 234 with both).
+constexpr int64_t kColSmallLanes = 150000;
+
 // Workgroups of k_col<S, L, OPS> resident on the current device at once (0 if
 // the runtime cannot say).  Queried once per kernel and device.
 template <int S, int L, bool OPS, int PV>
@@ -65,12 +74,35 @@ static hipError_t col_launch_v(const Geom& g, int nb, const Fields& fl, const Op
   return hipGetLastError();
 }
 
+// The small-grid form (k_col_small) where it applies: plan variant 0, the default
+// tile choice, few enough jobs, all groups' exchange buffers within 64 KiB.
+template <int S, bool OPS>
+static bool col_small_fits(const ColArgs& a) {
+  using C = ColCfg<S, col_lsmall2<S>()>;
+  const int groups = OPS ? a.njob : 1;
+  return groups <= (OPS ? kColSmallJobs : 1) && groups * C::NT <= 1024 && sizeof(float2) * C::LDS * groups <= 65536;
+}
+template <int S, bool OPS>
+static hipError_t col_launch_small(const Geom& g, int nb, const Fields& fl, const Ops& ops, const Inst* inst, const ColArgs& a,
+                                   hipStream_t st) {
+  constexpr int L = col_lsmall2<S>();
+  using C = ColCfg<S, L>;
+  const int groups = OPS ? a.njob : 1;
+  const dim3 grid(a.nouter * ((a.ncols + L - 1) / L), nb, OPS ? 1 : a.nbuf);
+  hipLaunchKernelGGL((k_col_small<S, L, OPS>), grid, dim3(C::NT * groups), sizeof(float2) * C::LDS * groups, st, g, fl, ops, inst, a);
+  return hipGetLastError();
+}
+
 // the plan variant a.pv where the length has one, variant 0 otherwise
 template <int S, int LW, bool OPS>
 static hipError_t col_launch(const Geom& g, int nb, const Fields& fl, const Ops& ops, const Inst* inst, const ColArgs& a,
                              hipStream_t st) {
   if constexpr (has_plan_variant(S)) {
-    if (a.pv) return col_launch_v<S, LW, OPS, 1>(g, nb, fl, ops, inst, a, st);
+    if (a.pv && a.small < 2) return col_launch_v<S, LW, OPS, 1>(g, nb, fl, ops, inst, a, st);
+  }
+  if (a.small && col_small_fits<S, OPS>(a)) {
+    const int64_t lanes = (int64_t)a.nouter * nb * a.ncols * FftShape<S>::TPL * (OPS ? a.njob : a.nbuf);
+    if (a.small == 2 || lanes <= kColSmallLanes) return col_launch_small<S, OPS>(g, nb, fl, ops, inst, a, st);
   }
   return col_launch_v<S, LW, OPS, 0>(g, nb, fl, ops, inst, a, st);
 }

@@ -21,8 +21,11 @@ namespace kw {
 
 __device__ __forceinline__ float2 cadd(float2 a, float2 b) { return make_float2(a.x + b.x, a.y + b.y); }
 __device__ __forceinline__ float2 csub(float2 a, float2 b) { return make_float2(a.x - b.x, a.y - b.y); }
+// The rounding of each component is spelled out: left to the compiler, which of the two
+// products a fused multiply-add rounds could differ from kernel to kernel, and forms of a
+// pass that a size rule switches between must give the same bits.
 __device__ __forceinline__ float2 cmul(float2 a, float2 b) {
-  return make_float2(a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x);
+  return make_float2(fmaf(a.x, b.x, -(a.y * b.y)), fmaf(a.x, b.y, a.y * b.x));
 }
 __device__ __forceinline__ float2 cscale(float2 a, float s) { return make_float2(a.x * s, a.y * s); }
 // multiply by -i (DIR=-1, forward) or +i (DIR=+1, inverse)
@@ -135,74 +138,79 @@ __device__ __forceinline__ void dft4(float2* v) {
   v[3] = csub(d02, d13);
 }
 
+// Fused multiply-adds in the butterflies are spelled out (see cmul).  The odd half of the
+// radix-8 butterfly adds first and scales by 1/sqrt(2) inside the last additions.
 template <int DIR>
 __device__ __forceinline__ void dft8(float2* v) {
   constexpr float h = 0.70710678118654752440f;
-  float2 a[8];
+  float2 e[4], o[4];
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
-    a[j] = cadd(v[j], v[j + 4]);
-    a[j + 4] = csub(v[j], v[j + 4]);
+    e[j] = cadd(v[j], v[j + 4]);
+    o[j] = csub(v[j], v[j + 4]);
   }
-  {
-    float2 t = a[5];
-    a[5] = DIR < 0 ? make_float2(h * (t.x + t.y), h * (t.y - t.x)) : make_float2(h * (t.x - t.y), h * (t.y + t.x));
-    a[6] = mul_dir_i<DIR>(a[6]);
-    t = a[7];
-    a[7] = DIR < 0 ? make_float2(h * (-t.x + t.y), h * (-t.y - t.x)) : make_float2(h * (-t.x - t.y), h * (-t.y + t.x));
-  }
-  float2 e[4] = {a[0], a[1], a[2], a[3]};
-  float2 o[4] = {a[4], a[5], a[6], a[7]};
   dft4<DIR>(e);
-  dft4<DIR>(o);
+  const float2 r2 = mul_dir_i<DIR>(o[2]);
+  const float2 s02 = cadd(o[0], r2), d02 = csub(o[0], r2);
+  // sqrt(2) times o1 and o3 turned by -+45 and -+135 degrees
+  const float2 p = DIR < 0 ? make_float2(o[1].x + o[1].y, o[1].y - o[1].x) : make_float2(o[1].x - o[1].y, o[1].y + o[1].x);
+  const float2 q = DIR < 0 ? make_float2(o[3].y - o[3].x, -o[3].y - o[3].x) : make_float2(-o[3].x - o[3].y, o[3].x - o[3].y);
+  const float2 s13 = cadd(p, q), d13 = mul_dir_i<DIR>(csub(p, q));
   v[0] = e[0]; v[2] = e[1]; v[4] = e[2]; v[6] = e[3];
-  v[1] = o[0]; v[3] = o[1]; v[5] = o[2]; v[7] = o[3];
+  v[1] = make_float2(fmaf(h, s13.x, s02.x), fmaf(h, s13.y, s02.y));
+  v[5] = make_float2(fmaf(-h, s13.x, s02.x), fmaf(-h, s13.y, s02.y));
+  v[3] = make_float2(fmaf(h, d13.x, d02.x), fmaf(h, d13.y, d02.y));
+  v[7] = make_float2(fmaf(-h, d13.x, d02.x), fmaf(-h, d13.y, d02.y));
 }
 
-template <int DIR>
-__device__ __forceinline__ void dft3(float2* v) {
-  constexpr float c = -0.5f;
-  constexpr float s = 0.86602540378443864676f;
-  float2 a0 = v[0], a1 = v[1], a2 = v[2];
-  float2 t1 = cadd(a1, a2);
-  float2 t2 = make_float2(a0.x + c * t1.x, a0.y + c * t1.y);
-  float2 d = csub(a1, a2);
-  float2 isd = DIR < 0 ? make_float2(s * d.y, -s * d.x) : make_float2(-s * d.y, s * d.x);
-  v[0] = cadd(a0, t1);
-  v[1] = cadd(t2, isd);
-  v[2] = csub(t2, isd);
-}
-
+// Odd radices from the sums and differences of the inputs j and R - j: outputs k and
+// R - k share their cosine part a and their sine part b, X_k = a -+ i b.
 template <int R, int DIR>
 __device__ __forceinline__ void dft_odd(float2* v) {
+  constexpr int H = (R - 1) / 2;
+  constexpr float c3[3] = {1.0f, -0.5f, -0.5f};
+  constexpr float s3[3] = {0.0f, 0.86602540378443864676f, -0.86602540378443864676f};
   constexpr float c5[5] = {1.0f, 0.30901699437494742f, -0.80901699437494742f, -0.80901699437494742f, 0.30901699437494742f};
   constexpr float s5[5] = {0.0f, 0.95105651629515357f, 0.58778525229247313f, -0.58778525229247313f, -0.95105651629515357f};
   constexpr float c7[7] = {1.0f, 0.62348980185873353f, -0.22252093395631440f, -0.90096886790241913f,
                            -0.90096886790241913f, -0.22252093395631440f, 0.62348980185873353f};
   constexpr float s7[7] = {0.0f, 0.78183148246802981f, 0.97492791218182361f, 0.43388373911755812f,
                            -0.43388373911755812f, -0.97492791218182361f, -0.78183148246802981f};
-  float2 in[R];
+  float2 p[H], d[H];
+  float2 sum = v[0];
 #pragma unroll
-  for (int j = 0; j < R; ++j) in[j] = v[j];
+  for (int j = 0; j < H; ++j) {
+    p[j] = cadd(v[j + 1], v[R - 1 - j]);
+    d[j] = csub(v[j + 1], v[R - 1 - j]);
+    sum = cadd(sum, p[j]);
+  }
+  const float2 x0 = v[0];
+  v[0] = sum;
 #pragma unroll
-  for (int k = 0; k < R; ++k) {
-    float2 acc = in[0];
+  for (int k = 1; k <= H; ++k) {
+    float2 a = x0, b = make_float2(0.f, 0.f);
 #pragma unroll
-    for (int j = 1; j < R; ++j) {
-      const int m = (j * k) % R;
-      const float cc = R == 5 ? c5[m] : c7[m];
-      const float ss = (R == 5 ? s5[m] : s7[m]) * (DIR < 0 ? -1.0f : 1.0f);
-      acc.x += in[j].x * cc - in[j].y * ss;
-      acc.y += in[j].x * ss + in[j].y * cc;
+    for (int j = 0; j < H; ++j) {
+      const int m = (k * (j + 1)) % R;
+      const float cc = R == 3 ? c3[m] : R == 5 ? c5[m] : c7[m];
+      const float ss = (R == 3 ? s3[m] : R == 5 ? s5[m] : s7[m]) * (DIR < 0 ? 1.0f : -1.0f);
+      a = make_float2(fmaf(cc, p[j].x, a.x), fmaf(cc, p[j].y, a.y));
+      b = j == 0 ? make_float2(ss * d[j].x, ss * d[j].y) : make_float2(fmaf(ss, d[j].x, b.x), fmaf(ss, d[j].y, b.y));
     }
-    v[k] = acc;
+    if constexpr (H == 1) {  // one product: it goes into the last addition
+      const float ss = s3[1] * (DIR < 0 ? 1.0f : -1.0f);
+      v[1] = make_float2(fmaf(ss, d[0].y, a.x), fmaf(-ss, d[0].x, a.y));
+      v[2] = make_float2(fmaf(-ss, d[0].y, a.x), fmaf(ss, d[0].x, a.y));
+    } else {
+      v[k] = make_float2(a.x + b.y, a.y - b.x);
+      v[R - k] = make_float2(a.x - b.y, a.y + b.x);
+    }
   }
 }
 
 template <int R, int DIR>
 __device__ __forceinline__ void dft(float2* v) {
   if constexpr (R == 2) dft2<DIR>(v);
-  else if constexpr (R == 3) dft3<DIR>(v);
   else if constexpr (R == 4) dft4<DIR>(v);
   else if constexpr (R == 8) dft8<DIR>(v);
   else dft_odd<R, DIR>(v);
@@ -297,8 +305,25 @@ struct FftShape {
   static_assert(N % E == 0, "elements per thread must divide the line length");
 };
 
+// Ordering of an exchange.  WS: every line of the exchange is owned by one wavefront
+// whose LDS operations complete in order, so only the compiler has to keep them in
+// place (several such wavefronts then share a workgroup without waiting for each
+// other); otherwise the workgroup barrier.
+template <bool WS>
+__device__ __forceinline__ void line_sync() {
+#ifdef __HIP__
+  if constexpr (WS) {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    return;
+  }
+#endif
+  __syncthreads();
+}
+
 // One stage on the owned elements v (see header); Idx maps (n, line) -> LDS slot.
-template <int N, int EM, int S, int DIR, class Idx, int PV = 0>
+template <int N, int EM, int S, int DIR, class Idx, int PV = 0, bool WS = false>
 __device__ __forceinline__ void reg_stage(float2 (&v)[(FftShape<N, EM, PV>::E)], float2* lds, const float2* __restrict__ tw, int c,
                                           int j0, const Idx& idx) {
   constexpr int E = FftShape<N, EM, PV>::E;
@@ -345,7 +370,7 @@ __device__ __forceinline__ void reg_stage(float2 (&v)[(FftShape<N, EM, PV>::E)],
     }
   }
   if constexpr (!LAST) {
-    __syncthreads();
+    line_sync<WS>();
     if constexpr (Idx::A > 0 && TPL % Idx::A == 0) {
       const int b = idx(j0, c);
 #pragma unroll
@@ -354,27 +379,35 @@ __device__ __forceinline__ void reg_stage(float2 (&v)[(FftShape<N, EM, PV>::E)],
 #pragma unroll
       for (int m = 0; m < E; ++m) v[m] = lds[idx(j0 + m * TPL, c)];
     }
-    __syncthreads();
+    line_sync<WS>();
   }
 }
 
-template <int N, int EM, int S, int DIR, class Idx, int PV = 0>
+template <int N, int EM, int S, int DIR, class Idx, int PV = 0, bool WS = false>
 __device__ __forceinline__ void reg_stages(float2 (&v)[(FftShape<N, EM, PV>::E)], float2* lds, const float2* __restrict__ tw, int c,
                                            int j0, const Idx& idx) {
   if constexpr (S < plan_nstages(N, PV)) {
-    reg_stage<N, EM, S, DIR, Idx, PV>(v, lds, tw, c, j0, idx);
-    reg_stages<N, EM, S + 1, DIR, Idx, PV>(v, lds, tw, c, j0, idx);
+    reg_stage<N, EM, S, DIR, Idx, PV, WS>(v, lds, tw, c, j0, idx);
+    reg_stages<N, EM, S + 1, DIR, Idx, PV, WS>(v, lds, tw, c, j0, idx);
   }
 }
 
 // Transform the owned elements of line c in place (natural order in, natural
 // order out at the same owned positions).  Every thread of the workgroup must
-// call it (it contains barriers); the LDS buffer must not be in use.
-template <int N, int DIR, class Idx, int EM = 1, int PV = 0>
+// call it (it contains barriers; WS: every thread of the wavefront, which owns
+// all lines of this LDS buffer); the LDS buffer must not be in use.
+template <int N, int DIR, class Idx, int EM = 1, int PV = 0, bool WS = false>
 __device__ __forceinline__ void fft_reg(float2 (&v)[(FftShape<N, EM, PV>::E)], float2* lds, const float2* __restrict__ tw, int c,
                                         int j0, const Idx& idx) {
   static_assert(plan_nstages(N, PV) > 0, "unsupported FFT length");
-  reg_stages<N, EM, 0, DIR, Idx, PV>(v, lds, tw, c, j0, idx);
+#ifdef __HIP_DEVICE_COMPILE__
+  // The caller's last products are rounded before the first butterflies add them: left
+  // open, whether the two contract into fused multiply-adds depends on the branches around
+  // them, so the forms of a pass could differ in the last bit.
+#pragma unroll
+  for (int m = 0; m < FftShape<N, EM, PV>::E; ++m) asm("" : "+v"(v[m].x), "+v"(v[m].y));
+#endif
+  reg_stages<N, EM, 0, DIR, Idx, PV, WS>(v, lds, tw, c, j0, idx);
 }
 
 }  // namespace kw

@@ -329,7 +329,7 @@ __global__ __launch_bounds__(kGenThreads) void k_gcol(Geom g, Fields fl, Ops ops
       {
         const float ky = gp(ops.k[1])[iy];
         kyz2 = ky * ky;
-        if (g.nd == 3) { const float kz = gp(ops.k[2])[iz]; kyz2 += kz * kz; }
+        if (g.nd == 3) { const float kz = gp(ops.k[2])[iz]; kyz2 = fmaf(kz, kz, kyz2); }
       }
       const float km2 = fmaf(kx, kx, kyz2);
       float2 op = make_float2(1.f, 0.f);

@@ -238,6 +238,9 @@ __device__ __forceinline__ void set_lane(float2 (&a)[E], int m, int h, float v) 
 #ifndef KW_WPE_COLOPS
 #define KW_WPE_COLOPS 4  // the prefetch of the next job input would take it to 130 VGPRs, 3 waves
 #endif
+#ifndef KW_COL_SMALL_MIN
+#define KW_COL_SMALL_MIN 2
+#endif
 #define KW_WPE(N, W) __attribute__((amdgpu_waves_per_eu((FftShape<N>::E <= 8 ? (W) : 1))))
 
 // Stage-ordered twiddles (kw_fft.hpp stage_tw_*) of an N-point plan from the
@@ -251,6 +254,41 @@ __device__ __forceinline__ void fill_stage_tw(float2* dst, const float2* src, in
     for (int e = tid; e < NS * (R - 1); e += nt) dst[B + e] = ld2(gp(src), (e % (R - 1) + 1) * (e / (R - 1)) * TWS);
     fill_stage_tw<N, PV, S + 1>(dst, src, tid, nt);
   }
+}
+
+// The same with a compile-time workgroup size: every load is issued before the first
+// LDS write, so their latencies overlap (small grids, where a kernel is one chain of
+// latencies).
+template <int N, int PV, int NT, int S = 1, int K = 0, int M>
+__device__ __forceinline__ void load_stage_tw(float2 (&r)[M], const float2* src, int tid) {
+  if constexpr (S < plan_nstages(N, PV)) {
+    constexpr int R = plan_stage_radix(N, S, PV), NS = plan_ns_before(N, S, PV);
+    constexpr int TWS = N / (NS * R), CNT = NS * (R - 1), IT = (CNT + NT - 1) / NT;
+#pragma unroll
+    for (int i = 0; i < IT; ++i) {
+      const int e = min(tid + i * NT, CNT - 1);
+      r[K + i] = ld2(gp(src), (e % (R - 1) + 1) * (e / (R - 1)) * TWS);
+    }
+    load_stage_tw<N, PV, NT, S + 1, K + IT>(r, src, tid);
+  }
+}
+template <int N, int PV, int NT, int S = 1, int K = 0, int M>
+__device__ __forceinline__ void put_stage_tw(const float2 (&r)[M], float2* dst, int tid) {
+  if constexpr (S < plan_nstages(N, PV)) {
+    constexpr int R = plan_stage_radix(N, S, PV), NS = plan_ns_before(N, S, PV);
+    constexpr int B = stage_tw_base<N, PV>(S), CNT = NS * (R - 1), IT = (CNT + NT - 1) / NT;
+#pragma unroll
+    for (int i = 0; i < IT; ++i)
+      if (tid + i * NT < CNT) dst[B + tid + i * NT] = r[K + i];
+    put_stage_tw<N, PV, NT, S + 1, K + IT>(r, dst, tid);
+  }
+}
+template <int N, int PV>
+constexpr int stage_tw_loads(int nt) {
+  int k = 0;
+  for (int s = 1; s < plan_nstages(N, PV); ++s)
+    k += (plan_ns_before(N, s, PV) * (plan_stage_radix(N, s, PV) - 1) + nt - 1) / nt;
+  return k < 1 ? 1 : k;
 }
 
 #define KW_ZPASS_PROLOGUE                                              \
@@ -900,7 +938,7 @@ __global__ __launch_bounds__((ColCfg<N, L, EM, PV>::NT)) KW_WPE(N, (OPS ? KW_WPE
     {
       const float ky = gp(ops.k[1])[iy];
       kyz2 = ky * ky;
-      if (g.nd == 3) { const float kz = gp(ops.k[2])[iz]; kyz2 += kz * kz; }
+      if (g.nd == 3) { const float kz = gp(ops.k[2])[iz]; kyz2 = fmaf(kz, kz, kyz2); }
     }
     float2 st[C::E];
     int cur_in = -1, pre_in = next_loaded ? a.job[0].in : -1;
@@ -994,6 +1032,117 @@ __global__ __launch_bounds__((ColCfg<N, L, EM, PV>::NT)) KW_WPE(N, (OPS ? KW_WPE
       }
     }
   }
+  }
+}
+
+// ---------------------------------------------------------------------------
+// column passes of small grids
+// ---------------------------------------------------------------------------
+// Where the tiles of k_col leave most of the chip idle, a pass is one chain of
+// latencies: load, transforms one job after the other, store.  This form shortens the
+// chain and gives the same bits: tiles of at most one or two wavefronts (col_lsmall2),
+// one group of lanes per job (each loads and transforms its job's input itself, so a
+// pass costs one forward and one inverse transform whatever its jobs; stores wait
+// until every group has read, since jobs may write each other's input) or per buffer
+// (blockIdx.z), and every load of the pass, operator values included, issued at once.
+constexpr int kColSmallJobs = 4;  // jobs of a small-grid pass (one group of lanes each)
+template <int N>
+constexpr int col_lsmall2() { return clampi(64 / FftShape<N>::TPL, KW_COL_SMALL_MIN, 32); }
+
+template <int N, int L, bool OPS>
+__global__ __launch_bounds__((ColCfg<N, L>::NT * (OPS ? kColSmallJobs : 1))) void k_col_small(Geom g, Fields fl, Ops ops, const Inst* __restrict__ inst, ColArgs a) {
+  using C = ColCfg<N, L>;
+  constexpr bool WS = C::NT == 64;
+  extern __shared__ float2 lds_all[];
+  __shared__ float2 twl[stage_tw_size<N>()];
+  const typename C::Idx idx{};
+  const int grp = OPS ? (int)threadIdx.x / C::NT : 0;
+  const int tid = threadIdx.x - grp * C::NT;
+  const int b = blockIdx.y;
+  float2* const lds = lds_all + grp * C::LDS;
+  const int ntile = (a.ncols + L - 1) / L;
+  const int lid = xcd_remap(blockIdx.x, gridDim.x);
+  const int o = lid / ntile, tile = lid % ntile;
+  const int c = tid % L, j0 = tid / L;
+  const int col = tile * L + c;
+  const bool valid = col < a.ncols;
+  const int64_t base = (int64_t)b * g.nspec + (int64_t)o * a.ostride + min(col, a.ncols - 1);
+  const XJob jb = OPS ? a.job[grp] : XJob{};
+  const int ibuf = OPS ? jb.in : a.bufs[blockIdx.z];
+  float2 v[C::E];
+  {
+    const auto src = gp(fl.spec[ibuf]);
+#pragma unroll
+    for (int m = 0; m < C::E; ++m) v[m] = ld2(src, base + (int64_t)(j0 + m * C::TPL) * a.estride);
+  }
+  constexpr int TW = stage_tw_loads<N, 0>(C::NT);
+  float2 twr[TW];
+  load_stage_tw<N, 0, C::NT>(twr, ops.tw[a.axis], tid);
+  // operator values of this lane's lines: the x wavenumbers, |k|^2 of the other axes, the job's
+  // x-axis vector or its per-column value
+  float kx[OPS ? C::E : 1], kyz2 = 0.f, kap = 0.f;
+  float2 opx[OPS ? C::E : 1], colv = make_float2(1.f, 0.f);
+  const float2* tab = nullptr;
+  if constexpr (OPS) {
+    const int colc = min(col, a.ncols - 1);
+    tab = jb.kind == XK_GRAD ? ops.grad[jb.axis] : jb.kind == XK_DIV ? ops.div[jb.axis] : jb.kind == XK_UNSTAGGER ? ops.unst[jb.axis] : nullptr;
+    kap = inst[b].kap;
+#pragma unroll
+    for (int m = 0; m < C::E; ++m) kx[m] = gp(ops.k[0])[j0 + m * C::TPL];
+    if (tab && jb.axis == 0) {
+#pragma unroll
+      for (int m = 0; m < C::E; ++m) opx[m] = ld2(gp(tab), j0 + m * C::TPL);
+    } else if (tab) {
+      colv = ld2(gp(tab), (jb.axis == 1 && g.nd == 3) ? o : colc);
+    }
+    const float ky = gp(ops.k[1])[g.nd == 2 ? (valid ? col : 0) : o];
+    kyz2 = ky * ky;
+    if (g.nd == 3) { const float kz = gp(ops.k[2])[valid ? col : 0]; kyz2 = fmaf(kz, kz, kyz2); }
+  }
+  if (fl.tdev && gp(fl.tdev)[b] >= inst[b].nt) return;
+  if (!valid) {
+#pragma unroll
+    for (int m = 0; m < C::E; ++m) v[m] = make_float2(0.f, 0.f);
+  }
+  if (grp == 0) put_stage_tw<N, 0, C::NT>(twr, twl, tid);
+  __syncthreads();
+  if constexpr (!OPS) {
+    if (a.mode == 0) fft_reg<N, -1, typename C::Idx, 1, 0, WS>(v, lds, twl, c, j0, idx);
+    else fft_reg<N, +1, typename C::Idx, 1, 0, WS>(v, lds, twl, c, j0, idx);
+  } else {
+    fft_reg<N, -1, typename C::Idx, 1, 0, WS>(v, lds, twl, c, j0, idx);
+    // the jobs next to this one on the same input (k_col: one common factor when all of
+    // them are gradients or divergences)
+    bool kgroup = true;
+    for (int i = grp; i >= 0 && a.job[i].in == jb.in; --i) kgroup &= a.job[i].kind == XK_GRAD || a.job[i].kind == XK_DIV;
+    for (int i = grp; i < a.njob && a.job[i].in == jb.in; ++i) kgroup &= a.job[i].kind == XK_GRAD || a.job[i].kind == XK_DIV;
+    const bool xtab = tab && jb.axis == 0;
+#pragma unroll
+    for (int m = 0; m < C::E; ++m) {
+      float2 op = xtab ? opx[m] : colv;
+      const float km2 = fmaf(kx[m], kx[m], kyz2);
+      if (kgroup) {
+        const float f = kap > 0.f ? sinc_k2(kap * kap * km2) : 1.f;
+        v[m] = cmul(cscale(v[m], f * ops.inv_ntot), op);
+        continue;
+      }
+      switch (jb.kind) {
+        case XK_GRAD:
+        case XK_DIV: op = cscale(op, kap > 0.f ? sinc_k2(kap * kap * km2) : 1.f); break;
+        case XK_FRAC1: op = make_float2(kpow2(km2, ops.frac1), 0.f); break;
+        case XK_FRAC2: op = make_float2(kpow2(km2, ops.frac2), 0.f); break;
+        case XK_SRCKAPPA: op = make_float2(kap > 0.f ? cos_k2(kap * kap * km2) : 1.f, 0.f); break;
+        default: break;
+      }
+      v[m] = cscale(cmul(v[m], op), ops.inv_ntot);
+    }
+    __syncthreads();  // every group has read its input
+    fft_reg<N, +1, typename C::Idx, 1, 0, WS>(v, lds, twl, c, j0, idx);
+  }
+  if (valid) {
+    const auto dst = gw(fl.spec[OPS ? jb.out : ibuf]);
+#pragma unroll
+    for (int m = 0; m < C::E; ++m) st2(dst, base + (int64_t)(j0 + m * C::TPL) * a.estride, v[m]);
   }
 }
 

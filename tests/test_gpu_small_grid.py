@@ -1,0 +1,70 @@
+"""The small-grid forms of the step kernels give the bits of the large-grid ones.
+
+A size rule switches between the two (kw_col_pass.hip), so a batch and its instances
+run alone, or a step before and after its sources end, may run different forms.
+"""
+import copy
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def _case(shape, absorb, bona):
+    """Multi-row pressure and velocity sources, heterogeneous medium, every record."""
+    from kwave_amd.data import Vector
+    from kwave_amd.kgrid import kWaveGrid
+    from kwave_amd.kmedium import kWaveMedium
+    from kwave_amd.ksensor import kSensor
+    from kwave_amd.ksource import kSource
+
+    rng = np.random.default_rng(11)
+    dx = 1e-4
+    kg = kWaveGrid(Vector(list(shape)), Vector([dx] * len(shape)))
+    kg.setTime(24, 0.3 * dx / 1700.0)
+    med = kWaveMedium(sound_speed=1500.0 + 200.0 * rng.random(shape), density=1000.0 + 50.0 * rng.random(shape))
+    if absorb:
+        med.alpha_coeff, med.alpha_power = absorb
+    if bona:
+        med.BonA = bona
+    src = kSource()
+    sl = tuple(slice(n // 2 - 2, n // 2 + 2) for n in shape)
+    pm = np.zeros(shape, dtype=bool)
+    pm[sl] = True
+    src.p_mask = src.u_mask = pm
+    n = int(pm.sum())
+    src.p = 1e4 * np.sin(0.4 * np.arange(12)[None, :] + 0.1 * np.arange(n)[:, None])
+    src.ux = 0.05 * np.cos(0.3 * np.arange(9)[None, :])
+    sm = np.zeros(shape, dtype=bool)
+    sm[tuple(slice(n // 4, 3 * n // 4) for n in shape[:-1]) + (slice(None, None, 3),)] = True
+    sen = kSensor(sm)
+    sen.record = ["p", "u_staggered", "p_final", "u_final"]
+    return kg, med, src, sen
+
+
+@pytest.mark.parametrize("shape,absorb,bona", [
+    ((16, 24), None, None),              # the shortest lines of each family
+    ((128, 128), None, None),
+    ((128, 40), (0.5, 1.3), 6.0),
+    ((512, 56), (0.02, 2.0), None),      # two wavefronts per tile
+    ((640, 16), (0.5, 1.5), None),
+    ((1024, 32), (0.5, 1.1), 6.0),       # the longest lines, four wavefronts per tile
+    ((24, 32, 40), (0.5, 1.3), 6.0),
+    ((48, 112, 16), None, 6.0),
+    ((32, 16, 768), (0.5, 1.5), None),
+])
+def test_small_grid_forms_give_the_same_bits(shape, absorb, bona, monkeypatch):
+    from kwave_amd.solvers.kspace_solver import Simulation
+
+    kg, med, src, sen = _case(shape, absorb, bona)
+
+    def run(small):
+        monkeypatch.setenv("KW_COL_SMALL", small)
+        return Simulation(kg, med, copy.deepcopy(src), sen, pml_size=(3,) * len(shape), pml_alpha=(2.0,) * len(shape)).run()
+
+    large = run("0")
+    assert all(np.abs(v).max() > 0 for v in large.values())
+    for form in ("1", "2"):
+        for k, v in run(form).items():
+            assert np.array_equal(v, large[k]), (form, k)
