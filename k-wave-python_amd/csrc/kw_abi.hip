@@ -436,6 +436,8 @@ int kw_plan_create(const kw_plan_desc* d, kw_plan** out) {
     // a caller that forces tile widths, radix plans or looping grids gets the passes those switches are for
     const char* sm = std::getenv("KW_COL_SMALL");
     const bool forced = P->col_wide || P->col_grid > 0 || std::getenv("KW_COL_TILES") || std::getenv("KW_COL_PLANS");
+    const char* zs = std::getenv("KW_Z_SMALL");
+    P->g.small = zs && zs[0] >= '0' && zs[0] <= '2' ? zs[0] - '0' : P->col_wide ? 0 : 1;
     P->col_small = sm && sm[0] >= '0' && sm[0] <= '2' ? sm[0] - '0' : forced ? 0 : 1;
   }
   int rc = KW_OK;

@@ -45,9 +45,9 @@ __global__ __launch_bounds__(ZCfg<N>::NT) void k_adj_eos(Geom g, Fields fl, AdjF
   const Inst& I = inst[b];
   float2 l1[ABS == 2 ? C::E : 1], l2[ABS == 2 ? C::E : 1];
   if constexpr (ABS == 2) {
-    inv_to_regs<N>(lds, fl.spec[0] + b * g.nspec, tw, row0, rows, g.nhp, tid, l1);
+    inv_to_regs<C>(lds, fl.spec[0] + b * g.nspec, tw, row0, rows, g.nhp, tid, l1);
     if (af.disp) {
-      inv_to_regs<N>(lds, fl.spec[1] + b * g.nspec, tw, row0, rows, g.nhp, tid, l2);
+      inv_to_regs<C>(lds, fl.spec[1] + b * g.nspec, tw, row0, rows, g.nhp, tid, l2);
     } else {
 #pragma unroll
       for (int m = 0; m < C::E; ++m) l2[m] = make_float2(0.f, 0.f);
@@ -142,7 +142,7 @@ __global__ __launch_bounds__(ZCfg<N>::NT) void k_adj_eos(Geom g, Fields fl, AdjF
       }
       w[m] = make_float2(wv[0], wv[1]);
     }
-    fwd_from_regs<N>(lds, w, fl.spec[i] + b * g.nspec, tw, row0, rows, g.nhp, tid);
+    fwd_from_regs<C>(lds, w, fl.spec[i] + b * g.nspec, tw, row0, rows, g.nhp, tid);
   }
   if (af.nonlin && inside) {
 #pragma unroll
@@ -199,8 +199,8 @@ __global__ __launch_bounds__(ZCfg<N>::NT) void k_adj_abs1(Geom g, Fields fl, Adj
     tw_v[m] = make_float2(tv[0], tv[1]);
     ew_v[m] = make_float2(ev[0], ev[1]);
   }
-  fwd_from_regs<N>(lds, tw_v, fl.spec[0] + b * g.nspec, tw, row0, rows, g.nhp, tid);
-  if (af.disp) fwd_from_regs<N>(lds, ew_v, fl.spec[1] + b * g.nspec, tw, row0, rows, g.nhp, tid);
+  fwd_from_regs<C>(lds, tw_v, fl.spec[0] + b * g.nspec, tw, row0, rows, g.nhp, tid);
+  if (af.disp) fwd_from_regs<C>(lds, ew_v, fl.spec[1] + b * g.nspec, tw, row0, rows, g.nhp, tid);
 }
 
 template <int N>
@@ -232,7 +232,7 @@ __global__ __launch_bounds__(ZCfg<N>::NT) void k_adj_mom(Geom g, Fields fl, AdjF
     dr[m] = make_float2(ld(I.dtr0[ax], i0, I.dtr0_s), ld(I.dtr0[ax], i0 + N, I.dtr0_s));
   }
   float2 gv[C::E];
-  inv_to_regs<N>(lds, sp, tw, row0, rows, g.nhp, tid, gv);
+  inv_to_regs<C>(lds, sp, tw, row0, rows, g.nhp, tid, gv);
 #pragma unroll
   for (int m = 0; m < C::E; ++m) {
     const float sz = zax ? pmlz[j0 + m * C::TPL] : 1.f;
@@ -255,7 +255,7 @@ __global__ __launch_bounds__(ZCfg<N>::NT) void k_adj_mom(Geom g, Fields fl, AdjF
     }
     gv[m] = make_float2(vv[0], vv[1]);
   }
-  fwd_from_regs<N>(lds, gv, sp, tw, row0, rows, g.nhp, tid);
+  fwd_from_regs<C>(lds, gv, sp, tw, row0, rows, g.nhp, tid);
 }
 
 template <int N, int ND>
@@ -270,7 +270,7 @@ __global__ __launch_bounds__(ZCfg<N>::NT) void k_adj_sum(Geom g, Fields fl, AdjF
 #pragma unroll
   for (int i = 0; i < ND; ++i) {
     float2 d[C::E];
-    inv_to_regs<N>(lds, fl.spec[i] + b * g.nspec, tw, row0, rows, g.nhp, tid, d);
+    inv_to_regs<C>(lds, fl.spec[i] + b * g.nspec, tw, row0, rows, g.nhp, tid, d);
 #pragma unroll
     for (int m = 0; m < C::E; ++m) {
       acc[m].x += d[m].x;

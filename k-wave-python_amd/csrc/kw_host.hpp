@@ -63,6 +63,7 @@ inline Geom make_geom(int nd, const int* n) {
   g.ntot = (int64_t)g.n[0] * g.n[1] * g.n[2];
   g.rows = (int)(g.ntot / g.nz);
   g.nspec = (int64_t)g.rows * g.nhp;
+  g.small = 1;
   return g;
 }
 

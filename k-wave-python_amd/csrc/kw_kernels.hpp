@@ -31,8 +31,11 @@ constexpr int clampi(int v, int lo, int hi) { return v < lo ? lo : (v > hi ? hi 
 #ifndef KW_ZPV
 #define KW_ZPV 0
 #endif
-template <int N>
+// NAR: the narrow form of small grids, one wavefront per workgroup (or per group of
+// lanes of a workgroup) where the line length leaves a wavefront room for it.
+template <int N_, bool NAR = false>
 struct ZCfg {
+  static constexpr int N = N_;
   // radix plan of the row passes: KW_ZPV=2 selects the radix-4 plan (4 elements per
   // thread) for power-of-two lengths
   static constexpr int PV = (KW_ZPV == 2 && (N & (N - 1)) == 0) ? 2 : 0;
@@ -40,9 +43,11 @@ struct ZCfg {
   static constexpr int E = F::E;
   static constexpr int TPL = F::TPL;
   static constexpr int L0 = clampi(pow2floor(2048 / N), 1, 64);
-  static constexpr int L = (L0 * TPL < 64) ? clampi(64 / TPL, L0, 64) : L0;  // row pairs per workgroup
+  static constexpr int L = NAR ? clampi(64 / TPL, 1, 64) : (L0 * TPL < 64) ? clampi(64 / TPL, L0, 64) : L0;  // row pairs per workgroup
   static constexpr int NT = TPL * L;
+  static constexpr bool WS = NAR && NT == 64;  // lines_sync without workgroup barriers
   static constexpr int NH = N / 2 + 1;
+  static constexpr int IT = (L * NH + NT - 1) / NT;  // spectrum values of a row per thread
   using Idx = RowIdx<N>;
   static constexpr int LDS = Idx::size(L);
 };
@@ -86,88 +91,110 @@ __device__ __forceinline__ float pml_at(const float* const* tab, const Geom& g, 
 }
 
 // Load the half spectra of the L row pairs of this workgroup into LDS as the
-// full spectrum of z = a + i b (Hermitian extension of each half spectrum).
-template <int N>
-__device__ __forceinline__ void load_pair_spec(float2* lds, const float2* __restrict__ spec_, int row0, int rows, int pitch, int tid) {
-  using C = ZCfg<N>;
-  const auto spec = gp(spec_);
+// full spectrum of z = a + i b (Hermitian extension of each half spectrum).  All of
+// a thread's loads (pair_load) are issued before its first LDS write (pair_put), so
+// their latencies overlap instead of adding up.
+template <class C>
+__device__ __forceinline__ void pair_put(float2* lds, const float2 (&As)[C::IT], const float2 (&Bs)[C::IT], int tid) {
+  constexpr int N = C::N;
   const typename C::Idx idx{};
-  // all of this thread's loads are issued before the first LDS write, so their
-  // latencies overlap instead of adding up
-  constexpr int IT = (C::L * C::NH + C::NT - 1) / C::NT;
-  float2 As[IT], Bs[IT];
 #pragma unroll
-  for (int it = 0; it < IT; ++it) {
+  for (int it = 0; it < C::IT; ++it) {
     const int e = tid + it * C::NT;
-    const int p = e / C::NH, k = e % C::NH;
-    const int ra = row0 + 2 * p, rb = ra + 1;
-    const bool in = e < C::L * C::NH;
-    As[it] = in && ra < rows ? ld2(spec, (int64_t)ra * pitch + k) : make_float2(0.f, 0.f);
-    Bs[it] = in && rb < rows ? ld2(spec, (int64_t)rb * pitch + k) : make_float2(0.f, 0.f);
-  }
-#pragma unroll
-  for (int it = 0; it < IT; ++it) {
-    const int e = tid + it * C::NT;
-    if (e >= C::L * C::NH) break;
+    if ((it + 1) * C::NT > C::L * C::NH && e >= C::L * C::NH) break;
     const int p = e / C::NH, k = e % C::NH;
     const float2 A = As[it], B = Bs[it];
-    if (k == 0 || (N % 2 == 0 && k == N / 2)) {
-      lds[idx(k, p)] = make_float2(A.x, B.x);
-    } else {
-      lds[idx(k, p)] = make_float2(A.x - B.y, A.y + B.x);
-      lds[idx(N - k, p)] = make_float2(A.x + B.y, B.x - A.y);
-    }
+    // the self-conjugate columns 0 and N/2 keep their real parts (both writes go to one slot)
+    const bool self = k == 0 || (N % 2 == 0 && k == N / 2);
+    const float2 lo = self ? make_float2(A.x, B.x) : make_float2(A.x - B.y, A.y + B.x);
+    const float2 hi = self ? lo : make_float2(A.x + B.y, B.x - A.y);
+    lds[idx(k, p)] = lo;
+    lds[idx(k == 0 ? 0 : N - k, p)] = hi;
+  }
+}
+
+// Rows (even in number) and columns are clamped into the grid rather than tested: a test
+// puts every load into a block of its own, which the compiler then waits for one by one.
+// What the clamped lanes read belongs to lines that are never stored.
+template <class C>
+__device__ __forceinline__ void pair_load(float2 (&As)[C::IT], float2 (&Bs)[C::IT], const float2* __restrict__ spec_, int row0, int rows,
+                                          int pitch, int tid) {
+  const auto spec = gp(spec_);
+#pragma unroll
+  for (int it = 0; it < C::IT; ++it) {
+    const int e = min(tid + it * C::NT, C::L * C::NH - 1);
+    const int p = e / C::NH, k = e % C::NH;
+    const int ra = min(row0 + 2 * p, rows - 2);
+    As[it] = ld2(spec, (int64_t)ra * pitch + k);
+    Bs[it] = ld2(spec, (int64_t)(ra + 1) * pitch + k);
   }
 }
 
 // After a forward FFT of z = a + i b (in LDS), split into the two half spectra.
-template <int N>
+template <class C>
 __device__ __forceinline__ void store_pair_spec(const float2* lds, float2* __restrict__ spec_, int row0, int rows, int pitch, int tid) {
-  using C = ZCfg<N>;
+  constexpr int N = C::N;
   const auto spec = gw(spec_);
   const typename C::Idx idx{};
-  for (int e = tid; e < C::L * C::NH; e += C::NT) {
+  float2 Z[C::IT], Zc[C::IT];
+#pragma unroll
+  for (int it = 0; it < C::IT; ++it) {
+    const int e = min(tid + it * C::NT, C::L * C::NH - 1);
     const int p = e / C::NH, k = e % C::NH;
-    const int ra = row0 + 2 * p, rb = ra + 1;
-    const float2 Z = lds[idx(k, p)];
-    const float2 Zc = lds[idx((N - k) % N, p)];
-    if (ra < rows) st2(spec, (int64_t)ra * pitch + k, make_float2(0.5f * (Z.x + Zc.x), 0.5f * (Z.y - Zc.y)));
-    if (rb < rows) st2(spec, (int64_t)rb * pitch + k, make_float2(0.5f * (Z.y + Zc.y), -0.5f * (Z.x - Zc.x)));
+    Z[it] = lds[idx(k, p)];
+    Zc[it] = lds[idx(k == 0 ? 0 : N - k, p)];
+  }
+#pragma unroll
+  for (int it = 0; it < C::IT; ++it) {
+    const int e = tid + it * C::NT;
+    const int p = e / C::NH, k = e % C::NH;
+    const int ra = row0 + 2 * p;  // both rows of a pair are inside the grid, or neither
+    if (((it + 1) * C::NT <= C::L * C::NH || e < C::L * C::NH) && ra < rows) {
+      st2(spec, (int64_t)ra * pitch + k, make_float2(0.5f * (Z[it].x + Zc[it].x), 0.5f * (Z[it].y - Zc[it].y)));
+      st2(spec, (int64_t)(ra + 1) * pitch + k, make_float2(0.5f * (Z[it].y + Zc[it].y), -0.5f * (Z[it].x - Zc[it].x)));
+    }
   }
 }
 
-// half spectra of a row pair -> real values of both rows at the owned positions
-template <int N>
-__device__ __forceinline__ void inv_to_regs(float2* lds, const float2* __restrict__ spec, const float2* __restrict__ tw,
-                                            int row0, int rows, int pitch, int tid, float2 (&out)[ZCfg<N>::E]) {
-  using C = ZCfg<N>;
+// full spectra of row pairs in LDS -> real values of both rows at the owned positions
+template <class C>
+__device__ __forceinline__ void inv_from_lds(float2* lds, const float2* __restrict__ tw, int tid, float2 (&out)[C::E]) {
   const typename C::Idx idx{};
   const int j0 = tid % C::TPL, c = tid / C::TPL;
-  __syncthreads();
-  load_pair_spec<N>(lds, spec, row0, rows, pitch, tid);
-  __syncthreads();
+  line_sync<C::WS>();
 #pragma unroll
   for (int m = 0; m < C::E; ++m) out[m] = lds[idx(j0 + m * C::TPL, c)];
-  __syncthreads();
-  fft_reg<N, +1, typename C::Idx, 1, C::PV>(out, lds, tw, c, j0, idx);
+  line_sync<C::WS>();
+  fft_reg<C::N, +1, typename C::Idx, 1, C::PV, C::WS>(out, lds, tw, c, j0, idx);
+}
+
+// half spectra of a row pair -> real values of both rows at the owned positions
+template <class C>
+__device__ __forceinline__ void inv_to_regs(float2* lds, const float2* __restrict__ spec, const float2* __restrict__ tw,
+                                            int row0, int rows, int pitch, int tid, float2 (&out)[C::E]) {
+  float2 As[C::IT], Bs[C::IT];
+  pair_load<C>(As, Bs, spec, row0, rows, pitch, tid);
+  line_sync<C::WS>();
+  pair_put<C>(lds, As, Bs, tid);
+  inv_from_lds<C>(lds, tw, tid, out);
 }
 
 // real values of a row pair at the owned positions -> half spectra of both rows
-template <int N>
-__device__ __forceinline__ void fwd_from_regs(float2* lds, float2 (&v)[ZCfg<N>::E], float2* __restrict__ spec,
-                                              const float2* __restrict__ tw, int row0, int rows, int pitch, int tid) {
-  using C = ZCfg<N>;
+// (stored where `store` holds)
+template <class C>
+__device__ __forceinline__ void fwd_from_regs(float2* lds, float2 (&v)[C::E], float2* __restrict__ spec,
+                                              const float2* __restrict__ tw, int row0, int rows, int pitch, int tid, bool store = true) {
   const typename C::Idx idx{};
   const int j0 = tid % C::TPL, c = tid / C::TPL;
-  fft_reg<N, -1, typename C::Idx, 1, C::PV>(v, lds, tw, c, j0, idx);
-  __syncthreads();
+  fft_reg<C::N, -1, typename C::Idx, 1, C::PV, C::WS>(v, lds, tw, c, j0, idx);
+  line_sync<C::WS>();
 #pragma unroll
   for (int m = 0; m < C::E; ++m) lds[idx(j0 + m * C::TPL, c)] = v[m];
-  __syncthreads();
-  store_pair_spec<N>(lds, spec, row0, rows, pitch, tid);
+  line_sync<C::WS>();
+  if (store) store_pair_spec<C>(lds, spec, row0, rows, pitch, tid);
   // leave the buffer free: a following transform writes it in its first stage
   // while slower waves could still be reading the pair spectra here
-  __syncthreads();
+  line_sync<C::WS>();
 }
 
 // Source value added/imposed at (row r, position n) for a CSR source term.
@@ -186,20 +213,47 @@ __device__ __forceinline__ bool csr_lookup(const Src& s, int r, int n, int t, fl
   return false;
 }
 
-// Source terms applied inside the unrolled element loops: the dense filtered
-// pattern (PATTERN, value sig(t) * pattern) and the inverse-transformed
-// multi-row source held in registers (CHAIN, value chv).  mode is SRC_NONE once
+// Filtered sources: the dense pattern (PATTERN, value sig(t) * pattern) and the
+// inverse transform of the multi-row source's spectrum (CHAIN).  mode is SRC_NONE once
 // the signal has ended.  The point-source modes (DIRICHLET, NOCORR) are applied
-// afterwards by a rolled pass over the owned source points (csr_apply), which
-// keeps their lookup out of the unrolled code.
+// afterwards by a rolled pass over the owned source points, which keeps their lookup
+// out of the unrolled code.
 __device__ __forceinline__ int src_mode_at(const Src& s, int t) { return t < s.len ? s.mode : SRC_NONE; }
 __device__ __forceinline__ float src_inline(const Src& s, int mode, float f, int64_t idx, float fac, float sig_t, float chv) {
-  if (mode == SRC_PATTERN) return f + fac * (sig_t * gp(s.pattern)[idx]);
-  if (mode == SRC_CHAIN) return f + fac * chv;
+  if (mode == SRC_PATTERN) return fmaf(fac, sig_t * gp(s.pattern)[idx], f);
+  if (mode == SRC_CHAIN) return fmaf(fac, chv, f);
   return f;
 }
+// the source values at a thread's elements (iA: its first element)
+template <class C>
+__device__ __forceinline__ void filtered_source(const Src& s, int mode, int t, int64_t iA, float2* lds, const Fields& fl, const Geom& g, int b,
+                                                const float2* tw, int row0, int rows, int tid, float2 (&ch)[C::E]) {
+  if (mode == SRC_CHAIN) {
+    inv_to_regs<C>(lds, fl.spec[s.chain_buf] + b * g.nspec, tw, row0, rows, g.nhp, tid, ch);
+  } else {
+    const float sig_t = gp(s.sig)[t];
+    const auto pat = gp(s.pattern);
+#pragma unroll
+    for (int m = 0; m < C::E; ++m) ch[m] = make_float2(sig_t * pat[iA + m * C::TPL], sig_t * pat[iA + C::N + m * C::TPL]);
+  }
+}
+template <class C>
+__device__ __forceinline__ void add_filtered_source(const Src& s, int mode, int t, float fac, int64_t iA, float2* lds, const Fields& fl,
+                                                    const Geom& g, int b, const float2* tw, int row0, int rows, int tid, float2 (&v)[C::E]) {
+  if (mode != SRC_CHAIN && mode != SRC_PATTERN) return;
+  float2 ch[C::E];
+  filtered_source<C>(s, mode, t, iA, lds, fl, g, b, tw, row0, rows, tid, ch);
+#pragma unroll
+  for (int m = 0; m < C::E; ++m) v[m] = make_float2(fmaf(fac, ch[m].x, v[m].x), fmaf(fac, ch[m].y, v[m].y));
+}
 __device__ __forceinline__ bool src_is_point(int mode) { return mode == SRC_DIRICHLET || mode == SRC_NOCORR; }
-__device__ __forceinline__ float src_point(int mode, float f, float fac, float v) { return mode == SRC_DIRICHLET ? fac * v : f + fac * v; }
+__device__ __forceinline__ float src_point(int mode, float f, float fac, float v) { return mode == SRC_DIRICHLET ? fac * v : fmaf(fac, v, f); }
+
+// PML-weighted update of a velocity or split-density component, s (s f - a b); the fused
+// multiply-add is spelled out so that every form of a step rounds alike (kw_fft.hpp, cmul).
+__device__ __forceinline__ float pml_update(float s, float f, float a, float b) { return s * fmaf(s, f, -(a * b)); }
+// A value other terms are added to is rounded here, not contracted into the addition.
+__device__ __forceinline__ void rounded(float& v) { asm("" : "+v"(v)); }
 
 // Register-array element (m, h) with a run-time m (selects, no indexed registers).
 template <int E>
@@ -219,10 +273,17 @@ __device__ __forceinline__ void set_lane(float2 (&a)[E], int m, int h, float v) 
 
 // Minimum waves per SIMD the register allocator must leave room for (kernels
 // with short register arrays only; 1 = unconstrained).  Measured at 512^3: every
-// floor that forces spills loses.  With the batched spectrum loads the mass kernel
-// runs 2409 us unconstrained (2 waves) against 2595 us forced to 3 (29 spilled
-// registers); the momentum kernel ran 1904 us at its natural 3 waves and 2808 us
-// forced to 4.
+// floor that forces spills loses (the mass kernel forced from 2 waves to 3 spilled 23
+// registers, 2155 -> 2948 us; the momentum kernel forced from 3 to 4, 1904 -> 2808 us).
+//
+// What bounds the updates on large grids is memory (512^3: mass 1686 us = 4.5 TB/s of
+// its algorithmic bytes, eos 811 us = 4.6, momentum 1846 us = 4.4; a plain copy reaches
+// 5.0), once their loads are issued in batches: element loops with a test inside (the
+// nonlinear flag, a source mode, a clamped row) had compiled into one block per element,
+// each load waited for alone.  Straight-line loops with the tests around them took the
+// mass kernel from 1970 to 1686 us at 512^3 and from 264 to 187 us at 256^3, eos from 902
+// to 811 and from 126 to 102 us, momentum from 198 to 186 us at 256^3 (1751 -> 1846 at
+// 512^3), and 256^3 steps from 1287 to 1159 us.
 #ifndef KW_WPE_MOM
 #define KW_WPE_MOM 1
 #endif
@@ -245,20 +306,8 @@ __device__ __forceinline__ void set_lane(float2 (&a)[E], int m, int h, float v) 
 
 // Stage-ordered twiddles (kw_fft.hpp stage_tw_*) of an N-point plan from the
 // natural table src[m] = exp(-2 pi i m / N), one stage at a time so that every
-// index is a compile-time expression of the entry.
-template <int N, int PV, int S = 1>
-__device__ __forceinline__ void fill_stage_tw(float2* dst, const float2* src, int tid, int nt) {
-  if constexpr (S < plan_nstages(N, PV)) {
-    constexpr int R = plan_stage_radix(N, S, PV), NS = plan_ns_before(N, S, PV);
-    constexpr int B = stage_tw_base<N, PV>(S), TWS = N / (NS * R);
-    for (int e = tid; e < NS * (R - 1); e += nt) dst[B + e] = ld2(gp(src), (e % (R - 1) + 1) * (e / (R - 1)) * TWS);
-    fill_stage_tw<N, PV, S + 1>(dst, src, tid, nt);
-  }
-}
-
-// The same with a compile-time workgroup size: every load is issued before the first
-// LDS write, so their latencies overlap (small grids, where a kernel is one chain of
-// latencies).
+// index is a compile-time expression of the entry; loads (into registers) and LDS
+// writes are separate, so that every load is in flight before the first write.
 template <int N, int PV, int NT, int S = 1, int K = 0, int M>
 __device__ __forceinline__ void load_stage_tw(float2 (&r)[M], const float2* src, int tid) {
   if constexpr (S < plan_nstages(N, PV)) {
@@ -291,12 +340,17 @@ constexpr int stage_tw_loads(int nt) {
   return k < 1 ? 1 : k;
 }
 
-#define KW_ZPASS_PROLOGUE                                              \
-  using C = ZCfg<N>;                                                   \
+#define KW_ZPASS_PROLOGUE KW_ZPASS_PROLOGUE_AS(ZCfg<N>)
+#define KW_ZPASS_PROLOGUE_AS(...)                                      \
+  using C = __VA_ARGS__;                                               \
   __shared__ float2 lds[C::LDS];                                       \
   __shared__ float2 twl[stage_tw_size<N, C::PV>()];                    \
   const int tid = threadIdx.x;                                         \
-  fill_stage_tw<N, C::PV>(twl, tw_g, tid, C::NT);                      \
+  {                                                                    \
+    float2 twr_[stage_tw_loads<N, C::PV>(C::NT)];                      \
+    load_stage_tw<N, C::PV, C::NT>(twr_, tw_g, tid);                   \
+    put_stage_tw<N, C::PV, C::NT>(twr_, twl, tid);                     \
+  }                                                                    \
   __syncthreads();                                                     \
   const float2* tw = twl;                                              \
   const int b = blockIdx.y;                                            \
@@ -306,30 +360,61 @@ constexpr int stage_tw_loads(int nt) {
   const int ra = row0 + 2 * pc;                                        \
   (void)j0; (void)ra;
 
+// The updates' prologue: the twiddles and the contiguous-axis PML (PTAB, or null) are
+// loaded into registers here and put into LDS by KW_ZPASS_PUT, once the kernel has
+// issued the loads of its operands and first spectrum (the transform's first barrier
+// publishes them).
+#define KW_ZPASS_EARLY(PTAB)                                           \
+  using C = ZCfg<N>;                                                   \
+  __shared__ float2 lds[C::LDS];                                       \
+  __shared__ float2 twl[stage_tw_size<N, C::PV>()];                    \
+  __shared__ float pmlz[N];                                            \
+  const int tid = threadIdx.x;                                         \
+  const int b = blockIdx.y;                                            \
+  const Inst& I = inst[b];                                             \
+  float2 twr[stage_tw_loads<N, C::PV>(C::NT)];                         \
+  load_stage_tw<N, C::PV, C::NT>(twr, tw_g, tid);                      \
+  constexpr int PZ = (N + C::NT - 1) / C::NT;                          \
+  float pzr[PZ];                                                       \
+  const float* const ptab = PTAB;                                      \
+  if (ptab) {                                                          \
+    _Pragma("unroll") for (int i_ = 0; i_ < PZ; ++i_) pzr[i_] = gp(ptab)[min(tid + i_ * C::NT, N - 1)]; \
+  }                                                                    \
+  const float2* tw = twl;                                              \
+  const int row0 = blockIdx.x * 2 * C::L;                              \
+  const int rows = g.rows;                                             \
+  const int j0 = tid % C::TPL, pc = tid / C::TPL;                      \
+  const int ra = row0 + 2 * pc;                                        \
+  (void)j0; (void)ra;
+#define KW_ZPASS_PUT                                                   \
+  put_stage_tw<N, C::PV, C::NT>(twr, twl, tid);                        \
+  if (ptab) {                                                          \
+    _Pragma("unroll") for (int i_ = 0; i_ < PZ; ++i_)                  \
+      if (tid + i_ * C::NT < N) pmlz[tid + i_ * C::NT] = pzr[i_];      \
+  }
+
 // ---------------------------------------------------------------------------
 // generic real <-> half-spectrum transforms along the contiguous axis
 // ---------------------------------------------------------------------------
-template <int N>
-__global__ __launch_bounds__(ZCfg<N>::NT) void k_zfwd(Geom g, const float* __restrict__ f, int64_t fstride, float2* __restrict__ spec,
+template <int N, bool NAR>
+__global__ __launch_bounds__((ZCfg<N, NAR>::NT)) void k_zfwd(Geom g, const float* __restrict__ f, int64_t fstride, float2* __restrict__ spec,
                                                       int64_t sstride, const float2* __restrict__ tw_g) {
-  KW_ZPASS_PROLOGUE
+  KW_ZPASS_PROLOGUE_AS(ZCfg<N, NAR>)
   const auto fb = gp(f + b * fstride);
   float2 v[C::E];
+  const int64_t iA = (int64_t)min(ra, rows - 2) * N + j0;  // row counts are even here
 #pragma unroll
-  for (int m = 0; m < C::E; ++m) {
-    const int n = j0 + m * C::TPL;
-    v[m] = make_float2(ra < rows ? fb[(int64_t)ra * N + n] : 0.f, ra + 1 < rows ? fb[(int64_t)(ra + 1) * N + n] : 0.f);
-  }
-  fwd_from_regs<N>(lds, v, spec + b * sstride, tw, row0, rows, g.nhp, tid);
+  for (int m = 0; m < C::E; ++m) v[m] = make_float2(fb[iA + m * C::TPL], fb[iA + N + m * C::TPL]);
+  fwd_from_regs<C>(lds, v, spec + b * sstride, tw, row0, rows, g.nhp, tid);
 }
 
-template <int N>
-__global__ __launch_bounds__(ZCfg<N>::NT) void k_zinv(Geom g, const float2* __restrict__ spec, int64_t sstride, float* __restrict__ f,
+template <int N, bool NAR>
+__global__ __launch_bounds__((ZCfg<N, NAR>::NT)) void k_zinv(Geom g, const float2* __restrict__ spec, int64_t sstride, float* __restrict__ f,
                                                       int64_t fstride, const float2* __restrict__ tw_g, float scale) {
-  KW_ZPASS_PROLOGUE
+  KW_ZPASS_PROLOGUE_AS(ZCfg<N, NAR>)
   const auto fb = gw(f + b * fstride);
   float2 v[C::E];
-  inv_to_regs<N>(lds, spec + b * sstride, tw, row0, rows, g.nhp, tid, v);
+  inv_to_regs<C>(lds, spec + b * sstride, tw, row0, rows, g.nhp, tid, v);
 #pragma unroll
   for (int m = 0; m < C::E; ++m) {
     const int n = j0 + m * C::TPL;
@@ -362,17 +447,10 @@ __device__ __forceinline__ void pml_rows(const float* const* tab, const Geom& g,
 // ---------------------------------------------------------------------------
 template <int N>
 __global__ __launch_bounds__(ZCfg<N>::NT) KW_WPE(N, KW_WPE_MOM) void k_momentum(Geom g, Fields fl, const Inst* __restrict__ inst, const float2* __restrict__ tw_g) {
-  KW_ZPASS_PROLOGUE
   const int ax = blockIdx.z;
-  const Inst& I = inst[b];
-  const int t = gp(fl.tdev)[b];
-  if (t >= I.nt) return;
-  // pml along the contiguous axis, staged next to the twiddles (read after the
-  // first barrier of the transform below)
-  __shared__ float pmlz[N];
   const bool zax = ax == g.nd - 1;
-  if (zax)
-    for (int i_ = tid; i_ < N; i_ += C::NT) pmlz[i_] = gp(I.pmlsg[ax])[i_];
+  KW_ZPASS_EARLY(zax ? inst[blockIdx.y].pmlsg[ax] : nullptr)
+  const int t = gp(fl.tdev)[b];
   KW_ROWS_CLAMPED
   float2* sp = fl.spec[ax] + b * g.nspec;
   const auto u = gw(fl.u[ax] + b * g.ntot);
@@ -387,31 +465,28 @@ __global__ __launch_bounds__(ZCfg<N>::NT) KW_WPE(N, KW_WPE_MOM) void k_momentum(
     uo[m] = make_float2(u[i0], u[i0 + N]);
     dr[m] = make_float2(ld(I.dtr0[ax], i0, I.dtr0_s), ld(I.dtr0[ax], i0 + N, I.dtr0_s));
   }
-  float2 gv[C::E];
-  inv_to_regs<N>(lds, sp, tw, row0, rows, g.nhp, tid, gv);
-  float2 ch[C::E];
+  float2 gv[C::E], As[C::IT], Bs[C::IT];
+  pair_load<C>(As, Bs, sp, row0, rows, g.nhp, tid);
+  if (t >= I.nt) return;
+  KW_ZPASS_PUT
+  pair_put<C>(lds, As, Bs, tid);
+  inv_from_lds<C>(lds, tw, tid, gv);
   const int smode = src_mode_at(src, t);
-  const bool chain = smode == SRC_CHAIN;
-  if (chain) inv_to_regs<N>(lds, fl.spec[src.chain_buf] + b * g.nspec, tw, row0, rows, g.nhp, tid, ch);
-  const float sig_t = smode == SRC_PATTERN ? gp(src.sig)[t] : 0.f;
+  // straight-line element loops: a test inside would split them into blocks whose loads
+  // and stores the compiler cannot move past each other
 #pragma unroll
   for (int m = 0; m < C::E; ++m) {
     const float sz = zax ? pmlz[j0 + m * C::TPL] : 1.f;
-    float res[2];
+    gv[m].x = pml_update(sz * ph[0], uo[m].x, dr[m].x, gv[m].x);
+    gv[m].y = pml_update(sz * ph[1], uo[m].y, dr[m].y, gv[m].y);
+  }
+  add_filtered_source<C>(src, smode, t, src.fac[ax], iA, lds, fl, g, b, tw, row0, rows, tid, gv);
+  if (inside) {
 #pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      const int64_t idx = iA + h * N + m * C::TPL;
-      const float s = sz * ph[h];
-      const float gval = h ? gv[m].y : gv[m].x;
-      float uv = s * (s * (h ? uo[m].y : uo[m].x) - (h ? dr[m].y : dr[m].x) * gval);
-      uv = src_inline(src, smode, uv, idx, src.fac[ax], sig_t, chain ? (h ? ch[m].y : ch[m].x) : 0.f);
-      res[h] = uv;
+    for (int m = 0; m < C::E; ++m) {
+      u[iA + m * C::TPL] = gv[m].x;
+      u[iA + N + m * C::TPL] = gv[m].y;
     }
-    if (inside) {
-      u[iA + m * C::TPL] = res[0];
-      u[iA + N + m * C::TPL] = res[1];
-    }
-    gv[m] = make_float2(res[0], res[1]);
   }
   if (src_is_point(smode) && inside) {
     for (int h = 0; h < 2; ++h) {
@@ -427,7 +502,7 @@ __global__ __launch_bounds__(ZCfg<N>::NT) KW_WPE(N, KW_WPE_MOM) void k_momentum(
       }
     }
   }
-  fwd_from_regs<N>(lds, gv, sp, tw, row0, rows, g.nhp, tid);
+  fwd_from_regs<C>(lds, gv, sp, tw, row0, rows, g.nhp, tid);
 }
 
 // ---------------------------------------------------------------------------
@@ -443,19 +518,13 @@ __global__ __launch_bounds__(ZCfg<N>::NT) KW_WPE(N, KW_WPE_MOM) void k_momentum(
 // ---------------------------------------------------------------------------
 template <int N, int ND, bool SREG, bool CAP>
 __global__ __launch_bounds__(ZCfg<N>::NT) KW_WPE(N, KW_WPE_MASS) void k_mass(Geom g, Fields fl, const Inst* __restrict__ inst, const float2* __restrict__ tw_g, int flags) {
-  KW_ZPASS_PROLOGUE
-  const Inst& I = inst[b];
+  KW_ZPASS_EARLY(inst[blockIdx.y].pml[ND - 1])
   const int t = gp(fl.tdev)[b];
-  if (t >= I.nt) return;
-  __shared__ float pmlz[N];  // pml along the contiguous axis (read after the first transform barrier)
-  for (int i_ = tid; i_ < N; i_ += C::NT) pmlz[i_] = gp(I.pml[ND - 1])[i_];
   KW_ROWS_CLAMPED
   const int64_t off = b * g.ntot;
   const Src& src = I.srcp;
   const int smode = src_mode_at(src, t);
-  const bool chain = SREG && smode == SRC_CHAIN;
-  const bool patt = SREG && smode == SRC_PATTERN;
-  const float sig_t = smode == SRC_PATTERN ? gp(src.sig)[t] : 0.f;
+  const bool filtered = SREG && (smode == SRC_CHAIN || smode == SRC_PATTERN);
   const bool powerlaw = flags & (FLAG_POWERLAW_ABS | FLAG_POWERLAW_DISP);
   float ph[ND][2];
 #pragma unroll
@@ -469,29 +538,35 @@ __global__ __launch_bounds__(ZCfg<N>::NT) KW_WPE(N, KW_WPE_MASS) void k_mass(Geo
   // large grids, about 4 bytes per voxel of extra HBM traffic; the 2-D kernels would drop
   // from three waves per SIMD to two, the mixed-radix ones from two to one.
   constexpr bool R0R = ND == 3 && C::E <= 16 && (N & (N - 1)) == 0;
+  // (Every loop below is straight-line over its elements, with tests around whole loops:
+  // a test inside puts each load into a block of its own that is waited for alone.)
   float2 qv[C::E], divu[C::E], rt[C::E], r0v[R0R ? C::E : 1];
   float2 ch[SREG ? C::E : 1];
 #pragma unroll
   for (int m = 0; m < C::E; ++m) {
     const int64_t i0 = iA + m * C::TPL;
-    float qa = ld(I.rho0, i0, I.rho0_s), qb = ld(I.rho0, i0 + N, I.rho0_s);
-    if constexpr (R0R) r0v[m] = make_float2(qa, qb);
-    if (flags & FLAG_NONLINEAR) {
-      qa += 2.f * gw(fl.rhot)[off + i0];
-      qb += 2.f * gw(fl.rhot)[off + i0 + N];
-    }
-    qv[m] = make_float2(I.dt * qa, I.dt * qb);
+    qv[m] = make_float2(ld(I.rho0, i0, I.rho0_s), ld(I.rho0, i0 + N, I.rho0_s));
+    if constexpr (R0R) r0v[m] = qv[m];
     divu[m] = make_float2(0.f, 0.f);
     rt[m] = make_float2(0.f, 0.f);
   }
-  if constexpr (SREG) {
-    if (chain) {
-      inv_to_regs<N>(lds, fl.spec[src.chain_buf] + b * g.nspec, tw, row0, rows, g.nhp, tid, ch);
-    } else if (patt) {
-      const auto pat = gp(src.pattern);
+  if (flags & FLAG_NONLINEAR) {
+    const auto rhot = gp(fl.rhot + off);
+    float2 ro[C::E];
 #pragma unroll
-      for (int m = 0; m < C::E; ++m) ch[m] = make_float2(sig_t * pat[iA + m * C::TPL], sig_t * pat[iA + N + m * C::TPL]);
-    }
+    for (int m = 0; m < C::E; ++m) ro[m] = make_float2(rhot[iA + m * C::TPL], rhot[iA + N + m * C::TPL]);
+#pragma unroll
+    for (int m = 0; m < C::E; ++m) qv[m] = make_float2(fmaf(2.f, ro[m].x, qv[m].x), fmaf(2.f, ro[m].y, qv[m].y));
+  }
+#pragma unroll
+  for (int m = 0; m < C::E; ++m) qv[m] = cscale(qv[m], I.dt);
+  float2 As[C::IT], Bs[C::IT];
+  pair_load<C>(As, Bs, fl.spec[0] + b * g.nspec, row0, rows, g.nhp, tid);
+  if (t >= I.nt) return;
+  KW_ZPASS_PUT
+  __syncthreads();
+  if constexpr (SREG) {
+    if (filtered) filtered_source<C>(src, smode, t, iA, lds, fl, g, b, tw, row0, rows, tid, ch);
   }
 #pragma unroll
   for (int i = 0; i < ND; ++i) {
@@ -499,13 +574,20 @@ __global__ __launch_bounds__(ZCfg<N>::NT) KW_WPE(N, KW_WPE_MASS) void k_mass(Geo
     // old split density, fetched before the transform so its latency overlaps it
     // (for short register arrays; the long mixed-radix ones load it in place)
     constexpr bool PF = C::E <= 16;
-    float2 ro[PF ? C::E : 1];
+    float2 ro[C::E];
     if constexpr (PF) {
 #pragma unroll
       for (int m = 0; m < C::E; ++m) ro[m] = make_float2(rho[iA + m * C::TPL], rho[iA + N + m * C::TPL]);
     }
     float2 d[C::E];
-    inv_to_regs<N>(lds, fl.spec[i] + b * g.nspec, tw, row0, rows, g.nhp, tid, d);
+    if (i > 0) pair_load<C>(As, Bs, fl.spec[i] + b * g.nspec, row0, rows, g.nhp, tid);
+    __syncthreads();
+    pair_put<C>(lds, As, Bs, tid);
+    inv_from_lds<C>(lds, tw, tid, d);
+    if constexpr (!PF) {
+#pragma unroll
+      for (int m = 0; m < C::E; ++m) ro[m] = make_float2(rho[iA + m * C::TPL], rho[iA + N + m * C::TPL]);
+    }
     if constexpr (CAP) {
       if (inside) {
         const auto dd = gw(fl.adjD + (int64_t)i * gridDim.y * g.ntot + off);
@@ -519,32 +601,28 @@ __global__ __launch_bounds__(ZCfg<N>::NT) KW_WPE(N, KW_WPE_MASS) void k_mass(Geo
 #pragma unroll
     for (int m = 0; m < C::E; ++m) {
       const float sz = (i == ND - 1) ? pmlz[j0 + m * C::TPL] : 1.f;
-      float res[2];
+      ro[m] = make_float2(pml_update(sz * ph[i][0], ro[m].x, qv[m].x, d[m].x), pml_update(sz * ph[i][1], ro[m].y, qv[m].y, d[m].y));
+    }
+    if constexpr (SREG) {
+      if (filtered) {
+        const float fac = src.fac[i];
 #pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        const int64_t idx = iA + h * N + m * C::TPL;
-        const float dv = h ? d[m].y : d[m].x;
-        const float s = sz * ph[i][h];
-        const float q = h ? qv[m].y : qv[m].x;
-        float rold;
-        if constexpr (PF) rold = h ? ro[m].y : ro[m].x;
-        else rold = rho[idx];
-        float rv = s * (s * rold - q * dv);
-        if constexpr (SREG) {
-          if (chain || patt) rv = rv + src.fac[i] * (h ? ch[m].y : ch[m].x);
-        } else {
-          rv = src_inline(src, smode, rv, idx, src.fac[i], sig_t, 0.f);
-        }
-        res[h] = rv;
+        for (int m = 0; m < C::E; ++m) ro[m] = make_float2(fmaf(fac, ch[m].x, ro[m].x), fmaf(fac, ch[m].y, ro[m].y));
       }
-      if (inside) {
-        rho[iA + m * C::TPL] = res[0];
-        rho[iA + N + m * C::TPL] = res[1];
+    }
+    if (inside) {
+#pragma unroll
+      for (int m = 0; m < C::E; ++m) {
+        rho[iA + m * C::TPL] = ro[m].x;
+        rho[iA + N + m * C::TPL] = ro[m].y;
       }
-      divu[m].x += d[m].x;
-      divu[m].y += d[m].y;
-      rt[m].x += res[0];
-      rt[m].y += res[1];
+    }
+#pragma unroll
+    for (int m = 0; m < C::E; ++m) {
+      rounded(ro[m].x);
+      rounded(ro[m].y);
+      divu[m] = cadd(divu[m], d[m]);
+      rt[m] = cadd(rt[m], ro[m]);
     }
   }
   if (src_is_point(smode) && inside) {
@@ -570,48 +648,70 @@ __global__ __launch_bounds__(ZCfg<N>::NT) KW_WPE(N, KW_WPE_MASS) void k_mass(Geo
       }
     }
   }
+  if (fl.rhot && inside) {
+    const auto rhot = gw(fl.rhot + off);
+#pragma unroll
+    for (int m = 0; m < C::E; ++m) {
+      rhot[iA + m * C::TPL] = rt[m].x;
+      rhot[iA + N + m * C::TPL] = rt[m].y;
+    }
+  }
+  float2 r0e[C::E];  // rho0 again: the lines this block read at its start, from L2 if still there
 #pragma unroll
   for (int m = 0; m < C::E; ++m) {
-    float a_out[2];
+    if constexpr (R0R) r0e[m] = r0v[m];
+    else r0e[m] = make_float2(ld(I.rho0, iA + m * C::TPL, I.rho0_s), ld(I.rho0, iA + N + m * C::TPL, I.rho0_s));
+  }
+  if (powerlaw) {
 #pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      const int64_t idx = iA + h * N + m * C::TPL;
-      float r0;
-      if constexpr (R0R) r0 = h ? r0v[m].y : r0v[m].x;
-      else r0 = ld(I.rho0, idx, I.rho0_s);  // the lines this block read at its start, from L2 if still there
-      const float du = h ? divu[m].y : divu[m].x;
-      const float rtv = h ? rt[m].y : rt[m].x;
-      if (powerlaw) {
-        a_out[h] = r0 * du;
-      } else {
-        float q = rtv;
-        const float c2 = ld(I.c0sq, idx, I.c0sq_s);
-        if (flags & FLAG_STOKES) {
-          q += tau_at(I, idx, c2) * r0 * du;
-          if (fl.adjA && inside) gw(fl.adjA)[off + idx] = r0 * du;  // adjoint replay: the Stokes operand
+    for (int m = 0; m < C::E; ++m) divu[m] = make_float2(r0e[m].x * divu[m].x, r0e[m].y * divu[m].y);
+  } else {
+    float2 c2v[C::E], q[C::E];
+#pragma unroll
+    for (int m = 0; m < C::E; ++m) {
+      const int64_t i0 = iA + m * C::TPL;
+      c2v[m] = make_float2(ld(I.c0sq, i0, I.c0sq_s), ld(I.c0sq, i0 + N, I.c0sq_s));
+      q[m] = rt[m];
+    }
+    if (flags & FLAG_STOKES) {
+#pragma unroll
+      for (int m = 0; m < C::E; ++m) {
+        const int64_t i0 = iA + m * C::TPL;
+        q[m].x = fmaf(tau_at(I, i0, c2v[m].x) * r0e[m].x, divu[m].x, q[m].x);
+        q[m].y = fmaf(tau_at(I, i0 + N, c2v[m].y) * r0e[m].y, divu[m].y, q[m].y);
+      }
+      if (fl.adjA && inside) {  // adjoint replay: the Stokes operand
+#pragma unroll
+        for (int m = 0; m < C::E; ++m) {
+          gw(fl.adjA)[off + iA + m * C::TPL] = r0e[m].x * divu[m].x;
+          gw(fl.adjA)[off + iA + N + m * C::TPL] = r0e[m].y * divu[m].y;
         }
-        if (flags & FLAG_NONLINEAR) q += ld(I.bona, idx, I.bona_s) * rtv * rtv / (2.f * r0);
-        a_out[h] = c2 * q;
       }
     }
+    if (flags & FLAG_NONLINEAR) {
+#pragma unroll
+      for (int m = 0; m < C::E; ++m) {
+        const int64_t i0 = iA + m * C::TPL;
+        q[m].x += ld(I.bona, i0, I.bona_s) * rt[m].x * rt[m].x / (2.f * r0e[m].x);
+        q[m].y += ld(I.bona, i0 + N, I.bona_s) * rt[m].y * rt[m].y / (2.f * r0e[m].y);
+      }
+    }
+#pragma unroll
+    for (int m = 0; m < C::E; ++m) divu[m] = make_float2(c2v[m].x * q[m].x, c2v[m].y * q[m].y);
     if (inside) {
-      const int64_t i0 = off + iA + m * C::TPL;
-      if (fl.rhot) {
-        gw(fl.rhot)[i0] = rt[m].x;
-        gw(fl.rhot)[i0 + N] = rt[m].y;
-      }
-      if (!powerlaw) {
-        gw(fl.p)[i0] = a_out[0];
-        gw(fl.p)[i0 + N] = a_out[1];
+      const auto p = gw(fl.p + off);
+#pragma unroll
+      for (int m = 0; m < C::E; ++m) {
+        p[iA + m * C::TPL] = divu[m].x;
+        p[iA + N + m * C::TPL] = divu[m].y;
       }
     }
-    divu[m] = make_float2(a_out[0], a_out[1]);
   }
   if (!powerlaw) {
-    fwd_from_regs<N>(lds, divu, fl.spec[0] + b * g.nspec, tw, row0, rows, g.nhp, tid);
+    fwd_from_regs<C>(lds, divu, fl.spec[0] + b * g.nspec, tw, row0, rows, g.nhp, tid);
   } else {
-    if (flags & FLAG_POWERLAW_ABS) fwd_from_regs<N>(lds, divu, fl.spec[0] + b * g.nspec, tw, row0, rows, g.nhp, tid);
-    if (flags & FLAG_POWERLAW_DISP) fwd_from_regs<N>(lds, rt, fl.spec[1] + b * g.nspec, tw, row0, rows, g.nhp, tid);
+    if (flags & FLAG_POWERLAW_ABS) fwd_from_regs<C>(lds, divu, fl.spec[0] + b * g.nspec, tw, row0, rows, g.nhp, tid);
+    if (flags & FLAG_POWERLAW_DISP) fwd_from_regs<C>(lds, rt, fl.spec[1] + b * g.nspec, tw, row0, rows, g.nhp, tid);
   }
 }
 
@@ -621,10 +721,8 @@ __global__ __launch_bounds__(ZCfg<N>::NT) KW_WPE(N, KW_WPE_MASS) void k_mass(Geo
 // ---------------------------------------------------------------------------
 template <int N>
 __global__ __launch_bounds__(ZCfg<N>::NT) KW_WPE(N, KW_WPE_EOS) void k_eos(Geom g, Fields fl, const Inst* __restrict__ inst, const float2* __restrict__ tw_g, int flags) {
-  KW_ZPASS_PROLOGUE
-  const Inst& I = inst[b];
+  KW_ZPASS_EARLY((const float*)nullptr)
   const int t = gp(fl.tdev)[b];
-  if (t >= I.nt) return;
   KW_ROWS_CLAMPED
   const int64_t off = b * g.ntot;
   const auto rhot = gw(fl.rhot + off);
@@ -635,9 +733,12 @@ __global__ __launch_bounds__(ZCfg<N>::NT) KW_WPE(N, KW_WPE_EOS) void k_eos(Geom 
     rtv[m] = make_float2(rhot[i0], rhot[i0 + N]);
     c2v[m] = make_float2(ld(I.c0sq, i0, I.c0sq_s), ld(I.c0sq, i0 + N, I.c0sq_s));
   }
+  if (t >= I.nt) return;
+  KW_ZPASS_PUT
+  __syncthreads();
   float2 av[C::E], bv[C::E];
-  if (flags & FLAG_POWERLAW_ABS) inv_to_regs<N>(lds, fl.spec[0] + b * g.nspec, tw, row0, rows, g.nhp, tid, av);
-  if (flags & FLAG_POWERLAW_DISP) inv_to_regs<N>(lds, fl.spec[1] + b * g.nspec, tw, row0, rows, g.nhp, tid, bv);
+  if (flags & FLAG_POWERLAW_ABS) inv_to_regs<C>(lds, fl.spec[0] + b * g.nspec, tw, row0, rows, g.nhp, tid, av);
+  if (flags & FLAG_POWERLAW_DISP) inv_to_regs<C>(lds, fl.spec[1] + b * g.nspec, tw, row0, rows, g.nhp, tid, bv);
   if (inside && fl.adjA && (flags & FLAG_POWERLAW_ABS)) {  // adjoint replay: keep the operands
 #pragma unroll
     for (int m = 0; m < C::E; ++m) {
@@ -652,27 +753,41 @@ __global__ __launch_bounds__(ZCfg<N>::NT) KW_WPE(N, KW_WPE_EOS) void k_eos(Geom 
       gw(fl.adjB)[off + iA + N + m * C::TPL] = bv[m].y;
     }
   }
+  float2 q[C::E];
 #pragma unroll
-  for (int m = 0; m < C::E; ++m) {
-    float out[2];
+  for (int m = 0; m < C::E; ++m) q[m] = rtv[m];
+  if (flags & FLAG_POWERLAW_ABS) {
 #pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      const int64_t idx = iA + h * N + m * C::TPL;
-      const float rt = h ? rtv[m].y : rtv[m].x;
-      const float c2 = h ? c2v[m].y : c2v[m].x;
-      float q = rt;
-      if (flags & FLAG_POWERLAW_ABS) q += tau_at(I, idx, c2) * (h ? av[m].y : av[m].x);
-      if (flags & FLAG_POWERLAW_DISP) q -= eta_at(I, idx, c2) * (h ? bv[m].y : bv[m].x);
-      if (flags & FLAG_NONLINEAR) q += ld(I.bona, idx, I.bona_s) * rt * rt / (2.f * ld(I.rho0, idx, I.rho0_s));
-      out[h] = c2 * q;
+    for (int m = 0; m < C::E; ++m) {
+      const int64_t i0 = iA + m * C::TPL;
+      q[m] = make_float2(fmaf(tau_at(I, i0, c2v[m].x), av[m].x, q[m].x), fmaf(tau_at(I, i0 + N, c2v[m].y), av[m].y, q[m].y));
     }
-    if (inside) {
-      gw(fl.p)[off + iA + m * C::TPL] = out[0];
-      gw(fl.p)[off + iA + N + m * C::TPL] = out[1];
-    }
-    av[m] = make_float2(out[0], out[1]);
   }
-  fwd_from_regs<N>(lds, av, fl.spec[0] + b * g.nspec, tw, row0, rows, g.nhp, tid);
+  if (flags & FLAG_POWERLAW_DISP) {
+#pragma unroll
+    for (int m = 0; m < C::E; ++m) {
+      const int64_t i0 = iA + m * C::TPL;
+      q[m] = make_float2(fmaf(-eta_at(I, i0, c2v[m].x), bv[m].x, q[m].x), fmaf(-eta_at(I, i0 + N, c2v[m].y), bv[m].y, q[m].y));
+    }
+  }
+  if (flags & FLAG_NONLINEAR) {
+#pragma unroll
+    for (int m = 0; m < C::E; ++m) {
+      const int64_t i0 = iA + m * C::TPL;
+      q[m].x += ld(I.bona, i0, I.bona_s) * rtv[m].x * rtv[m].x / (2.f * ld(I.rho0, i0, I.rho0_s));
+      q[m].y += ld(I.bona, i0 + N, I.bona_s) * rtv[m].y * rtv[m].y / (2.f * ld(I.rho0, i0 + N, I.rho0_s));
+    }
+  }
+#pragma unroll
+  for (int m = 0; m < C::E; ++m) av[m] = make_float2(c2v[m].x * q[m].x, c2v[m].y * q[m].y);
+  if (inside) {
+#pragma unroll
+    for (int m = 0; m < C::E; ++m) {
+      gw(fl.p)[off + iA + m * C::TPL] = av[m].x;
+      gw(fl.p)[off + iA + N + m * C::TPL] = av[m].y;
+    }
+  }
+  fwd_from_regs<C>(lds, av, fl.spec[0] + b * g.nspec, tw, row0, rows, g.nhp, tid);
 }
 
 // ---------------------------------------------------------------------------
@@ -685,7 +800,7 @@ __global__ __launch_bounds__(ZCfg<N>::NT) void k_init_u(Geom g, Fields fl, const
   const Inst& I = inst[b];
   const int64_t off = b * g.ntot;
   float2 gv[C::E];
-  inv_to_regs<N>(lds, fl.spec[ax] + b * g.nspec, tw, row0, rows, g.nhp, tid, gv);
+  inv_to_regs<C>(lds, fl.spec[ax] + b * g.nspec, tw, row0, rows, g.nhp, tid, gv);
 #pragma unroll
   for (int m = 0; m < C::E; ++m) {
     const int n = j0 + m * C::TPL;
@@ -713,9 +828,9 @@ __global__ __launch_bounds__(ZCfg<N>::NT) void k_init_u(Geom g, Fields fl, const
 // build the z-spectrum of a multi-row additive source at step t (mode CHAIN)
 // which = -1: pressure source, 0..2: velocity component
 // ---------------------------------------------------------------------------
-template <int N>
-__global__ __launch_bounds__(ZCfg<N>::NT) void k_src_build(Geom g, Fields fl, const Inst* __restrict__ inst, const float2* __restrict__ tw_g, int which) {
-  KW_ZPASS_PROLOGUE
+template <int N, bool NAR>
+__global__ __launch_bounds__((ZCfg<N, NAR>::NT)) void k_src_build(Geom g, Fields fl, const Inst* __restrict__ inst, const float2* __restrict__ tw_g, int which) {
+  KW_ZPASS_PROLOGUE_AS(ZCfg<N, NAR>)
   const Inst& I = inst[b];
   const int t = gp(fl.tdev)[b];
   const Src& s = which < 0 ? I.srcp : I.srcu[which];
@@ -747,7 +862,7 @@ __global__ __launch_bounds__(ZCfg<N>::NT) void k_src_build(Geom g, Fields fl, co
 #pragma unroll
   for (int m = 0; m < C::E; ++m) v[m] = lds[idx(j0 + m * C::TPL, pc)];
   __syncthreads();
-  fwd_from_regs<N>(lds, v, fl.spec[s.chain_buf] + b * g.nspec, tw, row0, rows, g.nhp, tid);
+  fwd_from_regs<C>(lds, v, fl.spec[s.chain_buf] + b * g.nspec, tw, row0, rows, g.nhp, tid);
 }
 
 // ---------------------------------------------------------------------------
@@ -760,11 +875,7 @@ __global__ __launch_bounds__(ZCfg<N>::NT) void k_src_build(Geom g, Fields fl, co
 // (no square root on the common path).  kappa = sinc(x) and cos(x) for
 // x = c_ref dt |k| / 2 from x^2: Taylor polynomials in x^2 up to x^2 = 4 (FP32
 // rounding), sin(x)/x and cos(x) beyond.
-__device__ __forceinline__ float sinc_k2(float x2) {
-  if (x2 > 4.f) {
-    const float x = sqrtf(x2);
-    return sinf(x) / x;
-  }
+__device__ __forceinline__ float sinc_poly(float x2) {
   float p = -1.f / 1307674368000.f;                 // -1/15!
   p = fmaf(p, x2, 1.f / 6227020800.f);              //  1/13!
   p = fmaf(p, x2, -1.f / 39916800.f);               // -1/11!
@@ -774,8 +885,14 @@ __device__ __forceinline__ float sinc_k2(float x2) {
   p = fmaf(p, x2, -1.f / 6.f);                      // -1/3!
   return fmaf(p, x2, 1.f);
 }
-__device__ __forceinline__ float cos_k2(float x2) {
-  if (x2 > 4.f) return cosf(sqrtf(x2));
+__device__ __forceinline__ float sinc_k2(float x2) {
+  if (x2 > 4.f) {
+    const float x = sqrtf(x2);
+    return sinf(x) / x;
+  }
+  return sinc_poly(x2);
+}
+__device__ __forceinline__ float cos_poly(float x2) {
   float p = -1.f / 87178291200.f;                   // -1/14!
   p = fmaf(p, x2, 1.f / 479001600.f);               //  1/12!
   p = fmaf(p, x2, -1.f / 3628800.f);                // -1/10!
@@ -785,8 +902,52 @@ __device__ __forceinline__ float cos_k2(float x2) {
   p = fmaf(p, x2, -0.5f);                           // -1/2!
   return fmaf(p, x2, 1.f);
 }
+__device__ __forceinline__ float cos_k2(float x2) { return x2 > 4.f ? cosf(sqrtf(x2)) : cos_poly(x2); }
 // |k|^a from |k|^2 for |k| > 0 (the fractional Laplacian is 0 at |k| = 0)
 __device__ __forceinline__ float kpow2(float km2, float a) { return km2 == 0.f ? 0.f : exp2f(0.5f * a * log2f(km2)); }
+
+// Spectral factor of a job at the lane's E elements: kappa(|k|) = sinc (GRAD, DIV; also
+// the common factor of an input whose jobs are all of these), cos (SRCKAPPA), the
+// fractional powers, 1 otherwise.  The kind and the range of the arguments are tested
+// around the loops, not per element: on any stable time step every argument is within
+// the polynomials' range (kx2max: the largest kx^2 of the axis), and the loops are
+// straight-line code.
+template <int E>
+__device__ __forceinline__ void job_factor(int kind, float kap, const float (&km2)[E], float kmax2, const Ops& ops, float (&f)[E]) {
+  if (kind == XK_FRAC1 || kind == XK_FRAC2) {
+    const float a = kind == XK_FRAC1 ? ops.frac1 : ops.frac2;
+#pragma unroll
+    for (int m = 0; m < E; ++m) f[m] = kpow2(km2[m], a);
+  } else if (kap > 0.f && (kind == XK_GRAD || kind == XK_DIV || kind == XK_SRCKAPPA)) {
+    const float k2 = kap * kap;
+    if (__any(k2 * kmax2 > 4.f)) {
+#pragma unroll
+      for (int m = 0; m < E; ++m) f[m] = kind == XK_SRCKAPPA ? cos_k2(k2 * km2[m]) : sinc_k2(k2 * km2[m]);
+    } else if (kind == XK_SRCKAPPA) {
+#pragma unroll
+      for (int m = 0; m < E; ++m) f[m] = cos_poly(k2 * km2[m]);
+    } else {
+#pragma unroll
+      for (int m = 0; m < E; ++m) f[m] = sinc_poly(k2 * km2[m]);
+    }
+  } else {
+#pragma unroll
+    for (int m = 0; m < E; ++m) f[m] = 1.f;
+  }
+}
+
+// v = st times a job's operator and 1/ntot: the tabled vector (in v) times its factor, or
+// the factor alone.
+template <int E>
+__device__ __forceinline__ void apply_job(bool tabled, const float2 (&st)[E], const float (&f)[E], float inv, float2 (&v)[E]) {
+  if (tabled) {
+#pragma unroll
+    for (int m = 0; m < E; ++m) v[m] = cscale(cmul(st[m], cscale(v[m], f[m])), inv);
+  } else {
+#pragma unroll
+    for (int m = 0; m < E; ++m) v[m] = cscale(cscale(st[m], f[m]), inv);
+  }
+}
 
 // Consecutive workgroup ids go to different XCDs (round robin over 8); give each
 // XCD a contiguous range of tiles so neighbouring tiles share its L2.
@@ -825,59 +986,64 @@ __global__ __launch_bounds__((ColCfg<N, L, EM, PV>::NT)) KW_WPE(N, (OPS ? KW_WPE
   const int tid = threadIdx.x;
   const int b = blockIdx.y;
   if (fl.tdev && gp(fl.tdev)[b] >= inst[b].nt) return;
-  fill_stage_tw<N, PV>(twl, ops.tw[a.axis], tid, C::NT);
+  {
+    float2 twr[stage_tw_loads<N, PV>(C::NT)];
+    load_stage_tw<N, PV, C::NT>(twr, ops.tw[a.axis], tid);
+    put_stage_tw<N, PV, C::NT>(twr, twl, tid);
+  }
   __syncthreads();
   const int ntile = (a.ncols + L - 1) / L;
   const int lid = xcd_remap(blockIdx.x, gridDim.x);
-  const int o = lid / ntile, tile = lid % ntile;
   const int c = tid % L, j0 = tid / L;
-  const int col = tile * L + c;
-  const bool valid = col < a.ncols;
-  const int64_t base = (int64_t)b * g.nspec + (int64_t)o * a.ostride + col;
   const float2* tw = twl;
+  const int ntiles = a.nouter * ntile;
+  // Tile lt: its lane's column, clamped into the spectrum (a lane beyond it transforms a
+  // copy of the last column and does not store it: tests around single loads would have
+  // the compiler wait for each alone).
+  auto tile_base = [&](int lt, bool& in) -> int64_t {
+    const int o = lt / ntile, col = (lt - o * ntile) * L + c;
+    in = col < a.ncols;
+    return (int64_t)b * g.nspec + (int64_t)o * a.ostride + min(col, a.ncols - 1) + (int64_t)j0 * a.estride;
+  };
+  const int64_t step = (int64_t)C::TPL * a.estride;
 
   float2 v[C::E];
   if constexpr (!OPS) {
     // software pipeline over the buffers and tiles: the loads of the next buffer
     // (after a tile's last buffer, the first buffer of this workgroup's next tile)
     // are in flight while the current one is transformed and stored
-    const int ntiles = a.nouter * ntile;
     float2 nx[C::E];
-    if (valid) {
+    bool vt = false;
+    int64_t bt = tile_base(min(lid, ntiles - 1), vt);
+    {
       const auto bp = gp(fl.spec[a.bufs[0]]);
 #pragma unroll
-      for (int m = 0; m < C::E; ++m) nx[m] = ld2(bp, base + (int64_t)(j0 + m * C::TPL) * a.estride);
+      for (int m = 0; m < C::E; ++m) nx[m] = ld2(bp, bt + m * step);
     }
     for (int lt = lid; lt < ntiles; lt += (int)gridDim.x) {
-      const int ot = lt / ntile, colt = (lt % ntile) * L + c;
-      const bool vt = colt < a.ncols;
-      const int64_t bt = (int64_t)b * g.nspec + (int64_t)ot * a.ostride + colt;
       const int ltn = lt + (int)gridDim.x;
-      const int coln = (ltn % ntile) * L + c;
-      const bool vn = ltn < ntiles && coln < a.ncols;
-      const int64_t bn = (int64_t)b * g.nspec + (int64_t)(ltn / ntile) * a.ostride + coln;
+      bool vn = false;
+      const int64_t bn = tile_base(min(ltn, ntiles - 1), vn);
       for (int q = 0; q < a.nbuf; ++q) {
         const auto bp = gw(fl.spec[a.bufs[q]]);
 #pragma unroll
-        for (int m = 0; m < C::E; ++m) v[m] = vt ? nx[m] : make_float2(0.f, 0.f);
-        if (q + 1 < a.nbuf) {
-          if (vt) {
-            const auto bq = gp(fl.spec[a.bufs[q + 1]]);
+        for (int m = 0; m < C::E; ++m) v[m] = nx[m];
+        if (q + 1 < a.nbuf || ltn < ntiles) {
+          const bool last = q + 1 == a.nbuf;
+          const auto bq = gp(fl.spec[a.bufs[last ? 0 : q + 1]]);
+          const int64_t bx = last ? bn : bt;
 #pragma unroll
-            for (int m = 0; m < C::E; ++m) nx[m] = ld2(bq, bt + (int64_t)(j0 + m * C::TPL) * a.estride);
-          }
-        } else if (vn) {
-          const auto bq = gp(fl.spec[a.bufs[0]]);
-#pragma unroll
-          for (int m = 0; m < C::E; ++m) nx[m] = ld2(bq, bn + (int64_t)(j0 + m * C::TPL) * a.estride);
+          for (int m = 0; m < C::E; ++m) nx[m] = ld2(bq, bx + m * step);
         }
         if (a.mode == 0) fft_reg<N, -1, typename C::Idx, EM, PV>(v, lds, tw, c, j0, idx);
         else fft_reg<N, +1, typename C::Idx, EM, PV>(v, lds, tw, c, j0, idx);
         if (vt) {
 #pragma unroll
-          for (int m = 0; m < C::E; ++m) st2(bp, bt + (int64_t)(j0 + m * C::TPL) * a.estride, v[m]);
+          for (int m = 0; m < C::E; ++m) st2(bp, bt + m * step, v[m]);
         }
       }
+      bt = bn;
+      vt = vn;
     }
   } else {
   // forward, multiply, inverse (outermost axis = axis 0), over the tiles lid,
@@ -905,7 +1071,7 @@ __global__ __launch_bounds__((ColCfg<N, L, EM, PV>::NT)) KW_WPE(N, (OPS ? KW_WPE
       for (int i_ = tid; i_ < N; i_ += C::NT) xop[slot][i_] = ld2(gp(t), i_);
     ++slot;
   }
-  const int ntiles = a.nouter * ntile;
+  const float kxe = gp(ops.k[0])[N / 2];  // the axis's largest wavenumber
   // The next distinct input is loaded while the current one is transformed and
   // its jobs stored: issued after those stores, its loads would also wait for
   // them (the vector-memory counter drains in order).  Within a tile, not when
@@ -918,8 +1084,8 @@ __global__ __launch_bounds__((ColCfg<N, L, EM, PV>::NT)) KW_WPE(N, (OPS ? KW_WPE
   for (int lt = lid; lt < ntiles; lt += (int)gridDim.x) {
     const int o = lt / ntile, tile = lt % ntile;
     const int col = tile * L + c;
-    const bool valid = col < a.ncols;
-    const int64_t base = (int64_t)b * g.nspec + (int64_t)o * a.ostride + col;
+    bool valid = false;
+    const int64_t base = tile_base(lt, valid);
     int iy, iz;
     if (g.nd == 2) { iy = valid ? col : 0; iz = 0; }
     else { iy = o; iz = valid ? col : 0; }
@@ -940,10 +1106,12 @@ __global__ __launch_bounds__((ColCfg<N, L, EM, PV>::NT)) KW_WPE(N, (OPS ? KW_WPE
       kyz2 = ky * ky;
       if (g.nd == 3) { const float kz = gp(ops.k[2])[iz]; kyz2 = fmaf(kz, kz, kyz2); }
     }
+    const float kmax2 = fmaf(kxe, kxe, kyz2);
     float2 st[C::E];
     int cur_in = -1, pre_in = next_loaded ? a.job[0].in : -1;
     bool kgroup = false;  // the current input's spectrum carries kappa / ntot
     next_loaded = false;
+    int slot = 0;  // x-table slot of the next x-axis job
     for (int j = 0; j < a.njob; ++j) {
       const XJob jb = a.job[j];
       if (jb.in != cur_in) {
@@ -954,29 +1122,33 @@ __global__ __launch_bounds__((ColCfg<N, L, EM, PV>::NT)) KW_WPE(N, (OPS ? KW_WPE
         } else {
           const auto src = gp(fl.spec[jb.in]);
 #pragma unroll
-          for (int m = 0; m < C::E; ++m) st[m] = valid ? ld2(src, base + (int64_t)(j0 + m * C::TPL) * a.estride) : make_float2(0.f, 0.f);
+          for (int m = 0; m < C::E; ++m) st[m] = ld2(src, base + m * step);
+          // wait here, not at the transform: there the compiler could not tell these loads
+          // from the ones issued ahead below and would wait for both
+#pragma unroll
+          for (int m = 0; m < C::E; ++m) asm volatile("" : "+v"(st[m].x), "+v"(st[m].y));
         }
         pre_in = -1;
         int k = j + 1;
         while (k < a.njob && a.job[k].in == cur_in) ++k;
-        if (PRE && k < a.njob) {
-          bool clobbered = false;
-          for (int i = j; i < k; ++i) clobbered |= a.job[i].out == a.job[k].in;
-          if (!clobbered) {
-            pre_in = a.job[k].in;
-            const auto nsrc = gp(fl.spec[pre_in]);
-#pragma unroll
-            for (int m = 0; m < C::E; ++m) nx[PRE ? m : 0] = valid ? ld2(nsrc, base + (int64_t)(j0 + m * C::TPL) * a.estride) : make_float2(0.f, 0.f);
+        if constexpr (PRE) {
+          int from = -1;  // what to load ahead
+          int64_t nbase = base;
+          if (k < a.njob) {
+            bool clobbered = false;
+            for (int i = j; i < k; ++i) clobbered |= a.job[i].out == a.job[k].in;
+            if (!clobbered) from = pre_in = a.job[k].in;
+          } else if (lt + (int)gridDim.x < ntiles) {
+            bool vn;
+            nbase = tile_base(lt + (int)gridDim.x, vn);
+            from = a.job[0].in;
+            next_loaded = true;
           }
-        } else if (PRE && lt + (int)gridDim.x < ntiles) {
-          const int ltn = lt + (int)gridDim.x;
-          const int on = ltn / ntile, coln = (ltn % ntile) * L + c;
-          const bool validn = coln < a.ncols;
-          const int64_t basen = (int64_t)b * g.nspec + (int64_t)on * a.ostride + coln;
-          const auto nsrc = gp(fl.spec[a.job[0].in]);
+          if (from >= 0) {
+            const auto nsrc = gp(fl.spec[from]);
 #pragma unroll
-          for (int m = 0; m < C::E; ++m) nx[PRE ? m : 0] = validn ? ld2(nsrc, basen + (int64_t)(j0 + m * C::TPL) * a.estride) : make_float2(0.f, 0.f);
-          next_loaded = true;
+            for (int m = 0; m < C::E; ++m) nx[m] = ld2(nsrc, nbase + m * step);
+          }
         }
         fft_reg<N, -1, typename C::Idx, EM, PV>(st, lds, tw, c, j0, idx);
         // When every job on this input is a gradient or divergence, the common
@@ -985,50 +1157,47 @@ __global__ __launch_bounds__((ColCfg<N, L, EM, PV>::NT)) KW_WPE(N, (OPS ? KW_WPE
         kgroup = true;
         for (int i = j; i < k; ++i) kgroup &= a.job[i].kind == XK_GRAD || a.job[i].kind == XK_DIV;
         if (kgroup) {
+          float km2[C::E], f[C::E];
 #pragma unroll
-          for (int m = 0; m < C::E; ++m) {
-            const float kx = kxs[j0 + m * C::TPL];
-            const float f = kap > 0.f ? sinc_k2(kap * kap * fmaf(kx, kx, kyz2)) : 1.f;
-            st[m] = cscale(st[m], f * ops.inv_ntot);
-          }
+          for (int m = 0; m < C::E; ++m) { const float kx = kxs[j0 + m * C::TPL]; km2[m] = fmaf(kx, kx, kyz2); }
+          job_factor(XK_GRAD, kap, km2, kmax2, ops, f);
+#pragma unroll
+          for (int m = 0; m < C::E; ++m) st[m] = cscale(st[m], f[m] * ops.inv_ntot);
         }
       }
-      // where this job's operator values live: an x-table slot, the per-column
-      // values, or (a third x-axis table) global memory
+      // where this job's operator values live: the per-column values, an x-table
+      // slot, or (a third x-axis table) global memory
       const bool tabled = jb.kind == XK_GRAD || jb.kind == XK_DIV || jb.kind == XK_UNSTAGGER;
-      int slot = 0;
-      for (int i = 0; i < j; ++i) {
-        const XJob q = a.job[i];
-        slot += q.axis == 0 && (q.kind == XK_GRAD || q.kind == XK_DIV || q.kind == XK_UNSTAGGER);
-      }
-      const float2* gtab = jb.kind == XK_GRAD ? ops.grad[0] : jb.kind == XK_DIV ? ops.div[0] : ops.unst[0];
-      const float2 colv = (tabled && jb.axis != 0) ? cop[j][c] : make_float2(1.f, 0.f);
+      if (tabled && jb.axis != 0) {
+        const float2 colv = cop[j][c];
 #pragma unroll
-      for (int m = 0; m < C::E; ++m) {
-        const int n = j0 + m * C::TPL;
-        float2 op = make_float2(1.f, 0.f);
-        if (tabled) op = jb.axis != 0 ? colv : (slot < 2 ? xop[slot][n] : ld2(gp(gtab), n));
-        if (kgroup) {
-          v[m] = cmul(st[m], op);
-          continue;
+        for (int m = 0; m < C::E; ++m) v[m] = colv;
+      } else if (tabled) {
+        if (slot < 2) {
+#pragma unroll
+          for (int m = 0; m < C::E; ++m) v[m] = xop[slot][j0 + m * C::TPL];
+        } else {
+          const auto gtab = gp(jb.kind == XK_GRAD ? ops.grad[0] : jb.kind == XK_DIV ? ops.div[0] : ops.unst[0]);
+#pragma unroll
+          for (int m = 0; m < C::E; ++m) v[m] = ld2(gtab, j0 + m * C::TPL);
         }
-        const float kx = kxs[n];
-        const float km2 = fmaf(kx, kx, kyz2);
-        switch (jb.kind) {
-          case XK_GRAD:
-          case XK_DIV: op = cscale(op, kap > 0.f ? sinc_k2(kap * kap * km2) : 1.f); break;  // kappa(|k|)
-          case XK_FRAC1: op = make_float2(kpow2(km2, ops.frac1), 0.f); break;
-          case XK_FRAC2: op = make_float2(kpow2(km2, ops.frac2), 0.f); break;
-          case XK_SRCKAPPA: op = make_float2(kap > 0.f ? cos_k2(kap * kap * km2) : 1.f, 0.f); break;
-          default: break;
-        }
-        v[m] = cscale(cmul(st[m], op), ops.inv_ntot);
+        ++slot;
+      }
+      if (kgroup) {
+#pragma unroll
+        for (int m = 0; m < C::E; ++m) v[m] = cmul(st[m], v[m]);
+      } else {
+        float km2[C::E], f[C::E];
+#pragma unroll
+        for (int m = 0; m < C::E; ++m) { const float kx = kxs[j0 + m * C::TPL]; km2[m] = fmaf(kx, kx, kyz2); }
+        job_factor(jb.kind, kap, km2, kmax2, ops, f);
+        apply_job<C::E>(tabled, st, f, ops.inv_ntot, v);
       }
       fft_reg<N, +1, typename C::Idx, EM, PV>(v, lds, tw, c, j0, idx);
       if (valid) {
         const auto dst = gw(fl.spec[jb.out]);
 #pragma unroll
-        for (int m = 0; m < C::E; ++m) st2(dst, base + (int64_t)(j0 + m * C::TPL) * a.estride, v[m]);
+        for (int m = 0; m < C::E; ++m) st2(dst, base + m * step, v[m]);
       }
     }
   }
@@ -1080,13 +1249,14 @@ __global__ __launch_bounds__((ColCfg<N, L>::NT * (OPS ? kColSmallJobs : 1))) voi
   load_stage_tw<N, 0, C::NT>(twr, ops.tw[a.axis], tid);
   // operator values of this lane's lines: the x wavenumbers, |k|^2 of the other axes, the job's
   // x-axis vector or its per-column value
-  float kx[OPS ? C::E : 1], kyz2 = 0.f, kap = 0.f;
+  float kx[OPS ? C::E : 1], kyz2 = 0.f, kap = 0.f, kxe = 0.f;
   float2 opx[OPS ? C::E : 1], colv = make_float2(1.f, 0.f);
   const float2* tab = nullptr;
   if constexpr (OPS) {
     const int colc = min(col, a.ncols - 1);
     tab = jb.kind == XK_GRAD ? ops.grad[jb.axis] : jb.kind == XK_DIV ? ops.div[jb.axis] : jb.kind == XK_UNSTAGGER ? ops.unst[jb.axis] : nullptr;
     kap = inst[b].kap;
+    kxe = gp(ops.k[0])[N / 2];
 #pragma unroll
     for (int m = 0; m < C::E; ++m) kx[m] = gp(ops.k[0])[j0 + m * C::TPL];
     if (tab && jb.axis == 0) {
@@ -1100,10 +1270,6 @@ __global__ __launch_bounds__((ColCfg<N, L>::NT * (OPS ? kColSmallJobs : 1))) voi
     if (g.nd == 3) { const float kz = gp(ops.k[2])[valid ? col : 0]; kyz2 = fmaf(kz, kz, kyz2); }
   }
   if (fl.tdev && gp(fl.tdev)[b] >= inst[b].nt) return;
-  if (!valid) {
-#pragma unroll
-    for (int m = 0; m < C::E; ++m) v[m] = make_float2(0.f, 0.f);
-  }
   if (grp == 0) put_stage_tw<N, 0, C::NT>(twr, twl, tid);
   __syncthreads();
   if constexpr (!OPS) {
@@ -1116,25 +1282,22 @@ __global__ __launch_bounds__((ColCfg<N, L>::NT * (OPS ? kColSmallJobs : 1))) voi
     bool kgroup = true;
     for (int i = grp; i >= 0 && a.job[i].in == jb.in; --i) kgroup &= a.job[i].kind == XK_GRAD || a.job[i].kind == XK_DIV;
     for (int i = grp; i < a.njob && a.job[i].in == jb.in; ++i) kgroup &= a.job[i].kind == XK_GRAD || a.job[i].kind == XK_DIV;
-    const bool xtab = tab && jb.axis == 0;
+    float km2[C::E], f[C::E];
 #pragma unroll
-    for (int m = 0; m < C::E; ++m) {
-      float2 op = xtab ? opx[m] : colv;
-      const float km2 = fmaf(kx[m], kx[m], kyz2);
-      if (kgroup) {
-        const float f = kap > 0.f ? sinc_k2(kap * kap * km2) : 1.f;
-        v[m] = cmul(cscale(v[m], f * ops.inv_ntot), op);
-        continue;
-      }
-      switch (jb.kind) {
-        case XK_GRAD:
-        case XK_DIV: op = cscale(op, kap > 0.f ? sinc_k2(kap * kap * km2) : 1.f); break;
-        case XK_FRAC1: op = make_float2(kpow2(km2, ops.frac1), 0.f); break;
-        case XK_FRAC2: op = make_float2(kpow2(km2, ops.frac2), 0.f); break;
-        case XK_SRCKAPPA: op = make_float2(kap > 0.f ? cos_k2(kap * kap * km2) : 1.f, 0.f); break;
-        default: break;
-      }
-      v[m] = cscale(cmul(v[m], op), ops.inv_ntot);
+    for (int m = 0; m < C::E; ++m) km2[m] = fmaf(kx[m], kx[m], kyz2);
+    job_factor(jb.kind, kap, km2, fmaf(kxe, kxe, kyz2), ops, f);
+    if (!(tab && jb.axis == 0)) {
+#pragma unroll
+      for (int m = 0; m < C::E; ++m) opx[m] = colv;
+    }
+    if (kgroup) {
+#pragma unroll
+      for (int m = 0; m < C::E; ++m) v[m] = cmul(cscale(v[m], f[m] * ops.inv_ntot), opx[m]);
+    } else {
+      float2 st[C::E];
+#pragma unroll
+      for (int m = 0; m < C::E; ++m) { st[m] = v[m]; v[m] = opx[m]; }
+      apply_job<C::E>(tab != nullptr, st, f, ops.inv_ntot, v);
     }
     __syncthreads();  // every group has read its input
     fft_reg<N, +1, typename C::Idx, 1, 0, WS>(v, lds, twl, c, j0, idx);
@@ -1144,6 +1307,327 @@ __global__ __launch_bounds__((ColCfg<N, L>::NT * (OPS ? kColSmallJobs : 1))) voi
 #pragma unroll
     for (int m = 0; m < C::E; ++m) st2(dst, base + (int64_t)(j0 + m * C::TPL) * a.estride, v[m]);
   }
+}
+
+// ---------------------------------------------------------------------------
+// contiguous-axis updates of small grids
+// ---------------------------------------------------------------------------
+// The updates above walk their axes one after the other on workgroups sized for
+// bandwidth; on a small grid that is a long chain of latencies on few compute units.
+// These forms give the same bits from one wavefront per row group and axis: the
+// transforms of the axes run side by side, their results meet once in LDS, every load
+// of the kernel is issued at its start, and a wavefront's exchanges need no workgroup
+// barrier (lines of 1024 take two wavefronts and keep the barriers).
+#define KW_ZSMALL_PROLOGUE(GROUPS)                                                                    \
+  using C = ZCfg<N, true>;                                                                            \
+  constexpr int G = GROUPS;                                                                           \
+  __shared__ float2 lds_all[G][C::LDS];                                                               \
+  __shared__ float2 twl[stage_tw_size<N, C::PV>()];                                                   \
+  const int grp = __builtin_amdgcn_readfirstlane((int)threadIdx.x / C::NT);                           \
+  const int tid = (int)threadIdx.x - grp * C::NT;                                                     \
+  float2* const lds = lds_all[grp];                                                                   \
+  const float2* tw = twl;                                                                             \
+  const int b = blockIdx.y;                                                                           \
+  const int row0 = blockIdx.x * 2 * C::L;                                                             \
+  const int rows = g.rows;                                                                            \
+  const int j0 = tid % C::TPL, pc = tid / C::TPL;                                                     \
+  const int ra = row0 + 2 * pc;                                                                       \
+  const Inst& I = inst[b];                                                                            \
+  constexpr int TWN = stage_tw_loads<N, C::PV>(G * C::NT);                                            \
+  float2 twr[TWN];
+
+// momentum (k_momentum): one group, blockIdx.z = axis
+template <int N>
+__global__ __launch_bounds__((ZCfg<N, true>::NT)) void k_momentum_small(Geom g, Fields fl, const Inst* __restrict__ inst, const float2* __restrict__ tw_g) {
+  KW_ZSMALL_PROLOGUE(1)
+  const int ax = blockIdx.z;
+  float2* const sp = fl.spec[ax] + b * g.nspec;
+  float2 As[C::IT], Bs[C::IT];
+  pair_load<C>(As, Bs, sp, row0, rows, g.nhp, tid);
+  load_stage_tw<N, C::PV, G * C::NT>(twr, tw_g, threadIdx.x);
+  const int t = gp(fl.tdev)[b];
+  KW_ROWS_CLAMPED
+  const auto u = gw(fl.u[ax] + b * g.ntot);
+  const Src& src = I.srcu[ax];
+  const bool zax = ax == g.nd - 1;
+  float2 uo[C::E], dr[C::E];
+  float pz[C::E], ph[2];
+#pragma unroll
+  for (int m = 0; m < C::E; ++m) {
+    const int64_t i0 = iA + m * C::TPL;
+    uo[m] = make_float2(u[i0], u[i0 + N]);
+    dr[m] = make_float2(ld(I.dtr0[ax], i0, I.dtr0_s), ld(I.dtr0[ax], i0 + N, I.dtr0_s));
+    pz[m] = 1.f;
+  }
+  if (zax) {
+#pragma unroll
+    for (int m = 0; m < C::E; ++m) pz[m] = gp(I.pmlsg[ax])[j0 + m * C::TPL];
+  }
+  pml_rows(I.pmlsg, g, ax, rA, ph);
+  if (t >= I.nt) return;
+  put_stage_tw<N, C::PV, G * C::NT>(twr, twl, threadIdx.x);
+  pair_put<C>(lds, As, Bs, tid);
+  float2 gv[C::E];
+  inv_from_lds<C>(lds, tw, tid, gv);
+  const int smode = src_mode_at(src, t);
+#pragma unroll
+  for (int m = 0; m < C::E; ++m) {
+    gv[m].x = pml_update(pz[m] * ph[0], uo[m].x, dr[m].x, gv[m].x);
+    gv[m].y = pml_update(pz[m] * ph[1], uo[m].y, dr[m].y, gv[m].y);
+  }
+  add_filtered_source<C>(src, smode, t, src.fac[ax], iA, lds, fl, g, b, tw, row0, rows, tid, gv);
+  if (inside) {
+#pragma unroll
+    for (int m = 0; m < C::E; ++m) {
+      u[iA + m * C::TPL] = gv[m].x;
+      u[iA + N + m * C::TPL] = gv[m].y;
+    }
+  }
+  if (src_is_point(smode) && inside) {
+    for (int h = 0; h < 2; ++h) {
+      const int r = ra + h;
+      if (gp(src.row_ptr)[r] == gp(src.row_ptr)[r + 1]) continue;
+      for (int m = 0; m < C::E; ++m) {
+        const int n = j0 + m * C::TPL;
+        float v;
+        if (!csr_lookup(src, r, n, t, v)) continue;
+        const float uv = src_point(smode, get_lane(gv, m, h), src.fac[ax], v);
+        u[(int64_t)r * N + n] = uv;
+        set_lane(gv, m, h, uv);
+      }
+    }
+  }
+  fwd_from_regs<C>(lds, gv, sp, tw, row0, rows, g.nhp, tid);
+}
+
+// mass conservation (k_mass): group i holds axis i; the divergence terms and the new split
+// densities of the axes meet in LDS and are added in axis order.  One form serves plans
+// with and without a filtered source and the adjoint replay (Fields::adjD).
+template <int N, int ND>
+__global__ __launch_bounds__((ZCfg<N, true>::NT * ND)) void k_mass_small(Geom g, Fields fl, const Inst* __restrict__ inst, const float2* __restrict__ tw_g, int flags) {
+  KW_ZSMALL_PROLOGUE(ND)
+  __shared__ float2 exd[ND][C::E * C::NT], exr[ND][C::E * C::NT];
+  float2 As[C::IT], Bs[C::IT];
+  pair_load<C>(As, Bs, fl.spec[grp] + b * g.nspec, row0, rows, g.nhp, tid);
+  load_stage_tw<N, C::PV, G * C::NT>(twr, tw_g, threadIdx.x);
+  const int t = gp(fl.tdev)[b];
+  KW_ROWS_CLAMPED
+  const int64_t off = b * g.ntot;
+  const Src& src = I.srcp;
+  const bool powerlaw = flags & (FLAG_POWERLAW_ABS | FLAG_POWERLAW_DISP);
+  const auto rho = gw(fl.rho[grp] + off);
+  float2 ro[C::E], r0v[C::E], qv[C::E], c2v[C::E];
+  float pz[C::E], ph[2];
+#pragma unroll
+  for (int m = 0; m < C::E; ++m) {
+    const int64_t i0 = iA + m * C::TPL;
+    ro[m] = make_float2(rho[i0], rho[i0 + N]);
+    r0v[m] = make_float2(ld(I.rho0, i0, I.rho0_s), ld(I.rho0, i0 + N, I.rho0_s));
+    c2v[m] = make_float2(ld(I.c0sq, i0, I.c0sq_s), ld(I.c0sq, i0 + N, I.c0sq_s));
+    pz[m] = 1.f;
+  }
+  if (flags & FLAG_NONLINEAR) {
+#pragma unroll
+    for (int m = 0; m < C::E; ++m) qv[m] = make_float2(gp(fl.rhot)[off + iA + m * C::TPL], gp(fl.rhot)[off + iA + N + m * C::TPL]);
+  }
+  if (grp == ND - 1) {
+#pragma unroll
+    for (int m = 0; m < C::E; ++m) pz[m] = gp(I.pml[ND - 1])[j0 + m * C::TPL];
+  }
+  pml_rows(I.pml, g, grp, rA, ph);
+  if (t >= I.nt) return;
+  const int smode = src_mode_at(src, t);
+  const bool filtered = smode == SRC_CHAIN || smode == SRC_PATTERN;
+  put_stage_tw<N, C::PV, G * C::NT>(twr, twl, threadIdx.x);
+  pair_put<C>(lds, As, Bs, tid);
+  __syncthreads();  // twiddles
+  float2 d[C::E], ch[C::E], res[C::E];
+  inv_from_lds<C>(lds, tw, tid, d);
+  if (filtered) filtered_source<C>(src, smode, t, iA, lds, fl, g, b, tw, row0, rows, tid, ch);
+  const float fac = src.fac[grp];
+  if (flags & FLAG_NONLINEAR) {
+#pragma unroll
+    for (int m = 0; m < C::E; ++m) qv[m] = make_float2(fmaf(2.f, qv[m].x, r0v[m].x), fmaf(2.f, qv[m].y, r0v[m].y));
+  } else {
+#pragma unroll
+    for (int m = 0; m < C::E; ++m) qv[m] = r0v[m];
+  }
+#pragma unroll
+  for (int m = 0; m < C::E; ++m)
+    res[m] = make_float2(pml_update(pz[m] * ph[0], ro[m].x, I.dt * qv[m].x, d[m].x), pml_update(pz[m] * ph[1], ro[m].y, I.dt * qv[m].y, d[m].y));
+  if (filtered) {
+#pragma unroll
+    for (int m = 0; m < C::E; ++m) res[m] = make_float2(fmaf(fac, ch[m].x, res[m].x), fmaf(fac, ch[m].y, res[m].y));
+  }
+  if (inside) {
+#pragma unroll
+    for (int m = 0; m < C::E; ++m) {
+      rho[iA + m * C::TPL] = res[m].x;
+      rho[iA + N + m * C::TPL] = res[m].y;
+    }
+  }
+  if (fl.adjD && inside) {  // adjoint replay: Dop_i u_i
+    const auto dd = gw(fl.adjD + (int64_t)grp * gridDim.y * g.ntot + off);
+#pragma unroll
+    for (int m = 0; m < C::E; ++m) {
+      dd[iA + m * C::TPL] = d[m].x;
+      dd[iA + N + m * C::TPL] = d[m].y;
+    }
+  }
+  if (src_is_point(smode) && inside) {
+    for (int h = 0; h < 2; ++h) {
+      const int r = ra + h;
+      if (gp(src.row_ptr)[r] == gp(src.row_ptr)[r + 1]) continue;
+      for (int m = 0; m < C::E; ++m) {
+        const int n = j0 + m * C::TPL;
+        float v;
+        if (!csr_lookup(src, r, n, t, v)) continue;
+        const float x = src_point(smode, get_lane(res, m, h), fac, v);
+        rho[(int64_t)r * N + n] = x;
+        set_lane(res, m, h, x);
+      }
+    }
+  }
+#pragma unroll
+  for (int m = 0; m < C::E; ++m) {
+    exd[grp][m * C::NT + tid] = d[m];
+    exr[grp][m * C::NT + tid] = res[m];
+  }
+  __syncthreads();
+  float2 divu[C::E], rt[C::E];
+#pragma unroll
+  for (int m = 0; m < C::E; ++m) {
+    float2 ds = make_float2(0.f, 0.f), rs = ds;
+#pragma unroll
+    for (int i = 0; i < ND; ++i) {
+      ds = cadd(ds, exd[i][m * C::NT + tid]);
+      rs = cadd(rs, exr[i][m * C::NT + tid]);
+    }
+    divu[m] = ds;
+    rt[m] = rs;
+  }
+  // group 0: p (or rho0 div u) and its transform; group 1: the density sum and, with
+  // dispersion, its transform
+  if (grp == 1 && fl.rhot && inside) {
+#pragma unroll
+    for (int m = 0; m < C::E; ++m) {
+      gw(fl.rhot)[off + iA + m * C::TPL] = rt[m].x;
+      gw(fl.rhot)[off + iA + N + m * C::TPL] = rt[m].y;
+    }
+  }
+  if (grp == 0) {
+#pragma unroll
+    for (int m = 0; m < C::E; ++m) {
+      float out[2];
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const int64_t idx = iA + h * N + m * C::TPL;
+        const float r0 = h ? r0v[m].y : r0v[m].x;
+        const float du = h ? divu[m].y : divu[m].x;
+        const float rtv = h ? rt[m].y : rt[m].x;
+        if (powerlaw) {
+          out[h] = r0 * du;
+        } else {
+          float q = rtv;
+          const float c2 = h ? c2v[m].y : c2v[m].x;
+          if (flags & FLAG_STOKES) {
+            q = fmaf(tau_at(I, idx, c2) * r0, du, q);
+            if (fl.adjA && inside) gw(fl.adjA)[off + idx] = r0 * du;
+          }
+          if (flags & FLAG_NONLINEAR) q += ld(I.bona, idx, I.bona_s) * rtv * rtv / (2.f * r0);
+          out[h] = c2 * q;
+        }
+      }
+      if (inside && !powerlaw) {
+        gw(fl.p)[off + iA + m * C::TPL] = out[0];
+        gw(fl.p)[off + iA + N + m * C::TPL] = out[1];
+      }
+      rt[m] = make_float2(out[0], out[1]);
+    }
+  }
+  const bool fwd = grp == 0 ? (!powerlaw || (flags & FLAG_POWERLAW_ABS)) : grp == 1 && (flags & FLAG_POWERLAW_DISP);
+  if (!C::WS || fwd) fwd_from_regs<C>(lds, rt, fl.spec[grp] + b * g.nspec, tw, row0, rows, g.nhp, tid, fwd);
+}
+
+// equation of state with power-law terms (k_eos): group 0 transforms the absorption
+// operand, group 1 the dispersion operand
+template <int N>
+__global__ __launch_bounds__((ZCfg<N, true>::NT * 2)) void k_eos_small(Geom g, Fields fl, const Inst* __restrict__ inst, const float2* __restrict__ tw_g, int flags) {
+  KW_ZSMALL_PROLOGUE(2)
+  __shared__ float2 ex[C::E * C::NT], exc[C::E * C::NT];
+  const bool abs = flags & FLAG_POWERLAW_ABS, disp = flags & FLAG_POWERLAW_DISP;
+  float2 As[C::IT], Bs[C::IT];
+  pair_load<C>(As, Bs, fl.spec[grp] + b * g.nspec, row0, rows, g.nhp, tid);
+  load_stage_tw<N, C::PV, G * C::NT>(twr, tw_g, threadIdx.x);
+  const int t = gp(fl.tdev)[b];
+  KW_ROWS_CLAMPED
+  const int64_t off = b * g.ntot;
+  float2 rtv[C::E], c2v[C::E], r0v[C::E], bav[C::E], co[C::E];
+#pragma unroll
+  for (int m = 0; m < C::E; ++m) {
+    const int64_t i0 = iA + m * C::TPL;
+    c2v[m] = make_float2(ld(I.c0sq, i0, I.c0sq_s), ld(I.c0sq, i0 + N, I.c0sq_s));
+    rtv[m] = make_float2(gp(fl.rhot)[off + i0], gp(fl.rhot)[off + i0 + N]);
+  }
+  if (flags & FLAG_NONLINEAR) {
+#pragma unroll
+    for (int m = 0; m < C::E; ++m) {
+      const int64_t i0 = iA + m * C::TPL;
+      r0v[m] = make_float2(ld(I.rho0, i0, I.rho0_s), ld(I.rho0, i0 + N, I.rho0_s));
+      bav[m] = make_float2(ld(I.bona, i0, I.bona_s), ld(I.bona, i0 + N, I.bona_s));
+    }
+  }
+  if (t >= I.nt) return;
+  put_stage_tw<N, C::PV, G * C::NT>(twr, twl, threadIdx.x);
+  pair_put<C>(lds, As, Bs, tid);
+  // this group's coefficient, tau or eta
+#pragma unroll
+  for (int m = 0; m < C::E; ++m) {
+    const int64_t i0 = iA + m * C::TPL;
+    if (grp == 0 && abs) co[m] = make_float2(tau_at(I, i0, c2v[m].x), tau_at(I, i0 + N, c2v[m].y));
+    if (grp == 1 && disp) co[m] = make_float2(eta_at(I, i0, c2v[m].x), eta_at(I, i0 + N, c2v[m].y));
+  }
+  __syncthreads();  // twiddles
+  float2 v[C::E];
+  inv_from_lds<C>(lds, tw, tid, v);
+  float* const keep = grp == 0 ? (abs ? fl.adjA : nullptr) : (disp ? fl.adjB : nullptr);
+  if (inside && keep) {  // adjoint replay: keep the operands
+#pragma unroll
+    for (int m = 0; m < C::E; ++m) {
+      gw(keep)[off + iA + m * C::TPL] = v[m].x;
+      gw(keep)[off + iA + N + m * C::TPL] = v[m].y;
+    }
+  }
+  if (grp == 1 && disp) {
+#pragma unroll
+    for (int m = 0; m < C::E; ++m) {
+      ex[m * C::NT + tid] = v[m];
+      exc[m * C::NT + tid] = co[m];
+    }
+  }
+  __syncthreads();
+  if (grp == 0) {
+#pragma unroll
+    for (int m = 0; m < C::E; ++m) {
+      const float2 bv = disp ? ex[m * C::NT + tid] : make_float2(0.f, 0.f), eta = disp ? exc[m * C::NT + tid] : make_float2(0.f, 0.f);
+      float out[2];
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const float rt = h ? rtv[m].y : rtv[m].x;
+        float q = rt;
+        if (abs) q = fmaf(h ? co[m].y : co[m].x, h ? v[m].y : v[m].x, q);
+        if (disp) q = fmaf(-(h ? eta.y : eta.x), h ? bv.y : bv.x, q);
+        if (flags & FLAG_NONLINEAR) q += (h ? bav[m].y : bav[m].x) * rt * rt / (2.f * (h ? r0v[m].y : r0v[m].x));
+        out[h] = (h ? c2v[m].y : c2v[m].x) * q;
+      }
+      if (inside) {
+        gw(fl.p)[off + iA + m * C::TPL] = out[0];
+        gw(fl.p)[off + iA + N + m * C::TPL] = out[1];
+      }
+      v[m] = make_float2(out[0], out[1]);
+    }
+  }
+  if (!C::WS || grp == 0) fwd_from_regs<C>(lds, v, fl.spec[0] + b * g.nspec, tw, row0, rows, g.nhp, tid, grp == 0);
 }
 
 // Supported line lengths, in four radix families.  Launcher files are compiled
@@ -1170,6 +1654,10 @@ inline bool size_supported_impl(int n) {
     default: return false;
   }
 }
+
+// Whether a contiguous-axis kernel takes its small-grid form: tpl lanes per row pair in
+// each of `groups` groups or grid layers (kw_dispatch.hip).
+bool z_small(const Geom& g, int nb, int tpl, int groups);
 
 inline dim3 zgrid(const Geom& g, int lpairs, int nb, int nz) {
   const int npairs = (g.rows + 1) / 2;

@@ -61,6 +61,7 @@ def test_small_grid_forms_give_the_same_bits(shape, absorb, bona, monkeypatch):
 
     def run(small):
         monkeypatch.setenv("KW_COL_SMALL", small)
+        monkeypatch.setenv("KW_Z_SMALL", small)
         return Simulation(kg, med, copy.deepcopy(src), sen, pml_size=(3,) * len(shape), pml_alpha=(2.0,) * len(shape)).run()
 
     large = run("0")
