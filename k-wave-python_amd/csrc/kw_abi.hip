@@ -205,7 +205,7 @@ int ev_get(kw_plan* P, size_t* idx) {
   } while (0)
 
 // y-pass over a list of buffers (3-D only)
-int ypass(kw_plan* P, int mode, const std::vector<int>& bufs) {
+int ypass(kw_plan* P, int mode, const std::vector<int>& bufs, int gath = 0) {
   if (P->g.nd != 3 || bufs.empty()) return KW_OK;
   ColArgs a = col_args(P->g, 1, mode);
   a.tile = P->col_tile[0];
@@ -214,6 +214,7 @@ int ypass(kw_plan* P, int mode, const std::vector<int>& bufs) {
   a.persist = P->col_persist;
   a.grid = P->col_grid;
   a.small = P->col_small;
+  a.gath = gath;
   a.nbuf = (int)bufs.size();
   for (size_t i = 0; i < bufs.size(); ++i) a.bufs[i] = bufs[i];
   const double spec_bytes = 8.0 * P->nb * (double)P->g.rows * P->g.nh;
@@ -221,7 +222,7 @@ int ypass(kw_plan* P, int mode, const std::vector<int>& bufs) {
   return KW_OK;
 }
 
-int xpass(kw_plan* P, const std::vector<XJob>& jobs, int kind) {
+int xpass(kw_plan* P, const std::vector<XJob>& jobs, int kind, int gath = 0) {
   ColArgs a = col_args(P->g, 0, 2);
   a.tile = P->col_tile[1];
   a.pv = P->col_pv[1];
@@ -229,6 +230,7 @@ int xpass(kw_plan* P, const std::vector<XJob>& jobs, int kind) {
   a.persist = P->col_persist;
   a.grid = P->col_grid;
   a.small = P->col_small;
+  a.gath = gath;
   a.njob = (int)jobs.size();
   int nin = 0, last = -1;
   for (size_t i = 0; i < jobs.size(); ++i) {
@@ -276,11 +278,18 @@ double zbytes_eos(const kw_plan* P) {
 // One time step.  lean: every spectral (CHAIN) and pattern pressure source
 // has ended, so no source spectrum is built or carried through the column
 // passes and the mass update takes its form without a staged source term.
-int enqueue_step(kw_plan* P, bool lean = false) {
+//
+// Step j of a block of k: the device step counters stand at the block's first step and
+// are advanced once, by k, at its end.  Every step after the block's first gathers the
+// sensors of the step before it in its first column pass (ColArgs::gath); the last
+// gathers its own before the counters advance, so a block leaves nothing behind.
+int enqueue_step(kw_plan* P, bool lean = false, int j = 0, int k = 1) {
   const Geom& g = P->g;
   const int D = g.nd;
   const float2* twz = P->ops.tw[D - 1];
   int rc;
+  P->fl.toff = j;
+  const int gath = j > 0 && !P->skip_gather ? P->max_sens : 0;
   // --- momentum: grad p, u update, F_z[u_i] ---
   std::vector<int> ub;
   std::vector<XJob> jobs;
@@ -293,8 +302,8 @@ int enqueue_step(kw_plan* P, bool lean = false) {
     }
   std::vector<int> y0 = {0};
   y0.insert(y0.end(), ub.begin(), ub.end());
-  if ((rc = ypass(P, 0, y0))) return rc;
-  if ((rc = xpass(P, jobs, KK_XGRAD))) return rc;
+  if ((rc = ypass(P, 0, y0, gath))) return rc;
+  if ((rc = xpass(P, jobs, KK_XGRAD, D == 2 ? gath : 0))) return rc;
   std::vector<int> y1;
   for (int i = 0; i < D; ++i) y1.push_back(i);
   y1.insert(y1.end(), ub.begin(), ub.end());
@@ -331,8 +340,11 @@ int enqueue_step(kw_plan* P, bool lean = false) {
     if ((rc = ypass(P, 1, yb))) return rc;
     KW_TLAUNCH(KK_EOS, zbytes_eos(P), launch_eos(g, P->nb, P->fl, P->d_inst, twz, P->flags, P->st));
   }
-  if (!P->skip_gather) KW_TLAUNCH(KK_GATHER, 0.0, launch_gather(g, P->nb, P->max_sens, P->fl, P->d_inst, P->st));
-  KW_TLAUNCH(KK_TICK, 0.0, launch_tick(P->fl, P->d_inst, P->nb, P->st));
+  if (j == k - 1) {
+    if (P->skip_gather) KW_TLAUNCH(KK_TICK, 0.0, launch_tick(P->fl, P->d_inst, P->nb, k, P->st));
+    else KW_TLAUNCH(KK_GATHER, 0.0, launch_gather_tick(g, P->nb, P->max_sens, P->fl, P->d_inst, k, P->st));
+  }
+  P->fl.toff = 0;
   return KW_OK;
 }
 
@@ -342,7 +354,7 @@ int build_graphs(kw_plan* P) {
     const int nsteps = pass % 2 == 0 ? 1 : P->graph_k;
     KW_HIP(hipStreamBeginCapture(P->st, hipStreamCaptureModeThreadLocal));
     int rc = KW_OK;
-    for (int s = 0; s < nsteps && rc == KW_OK; ++s) rc = enqueue_step(P, pass >= 2);
+    for (int s = 0; s < nsteps && rc == KW_OK; ++s) rc = enqueue_step(P, pass >= 2, s, nsteps);
     hipGraph_t graph = nullptr;
     hipError_t e = hipStreamEndCapture(P->st, &graph);
     if (rc) { if (graph) (void)hipGraphDestroy(graph); return rc; }
@@ -761,6 +773,12 @@ int autotune_tiles(kw_plan* P) {
   // >= 3 % faster
   for (int kind = 0; kind < 2 && rc == KW_OK; ++kind) {
     const int nline = (kind == 1 || D == 2) ? g.n[0] : g.n[1];
+    // the generic family and the small-grid form have tiles of their own
+    if (!ftile && !fpv) {
+      ColArgs a = col_args(g, kind == 1 || D == 2 ? 0 : 1, kind == 1 ? 2 : 0);
+      a.njob = a.nbuf = D;
+      if (!compiled_size(nline) || (P->col_small && col_small_lanes(a, nline, P->nb) <= kColSmallLanes)) continue;
+    }
     const int npv = tune_pv && compiled_size(nline) && has_plan_variant(nline) ? 2 : 1;
     // a forced choice is the only candidate of its kind
     const int pv0 = fpv ? P->col_pv[kind] : 0, pv1 = fpv ? P->col_pv[kind] + 1 : npv;
@@ -830,6 +848,7 @@ int kw_plan_init(kw_plan* P) {
   if (!P) return fail(KW_EINVAL, "NULL plan");
   KW_HIP(hipSetDevice(P->dev));
   P->t_host = -1;
+  P->fl.toff = 0;
   const Geom& g = P->g;
   int with_p0 = 0;
   for (int b = 0; b < P->nb; ++b) {
@@ -888,7 +907,7 @@ int kw_plan_init(kw_plan* P) {
     }
     KW_LAUNCH(launch_zfwd(g, P->nb, P->fl.p, g.ntot, P->fl.spec[0], g.nspec, twz, P->st));
     KW_LAUNCH(launch_gather(g, P->nb, P->max_sens, P->fl, P->d_inst, P->st));
-    KW_LAUNCH(launch_tick(P->fl, P->d_inst, P->nb, P->st));
+    KW_LAUNCH(launch_tick(P->fl, P->d_inst, P->nb, 1, P->st));
   }
   KW_HIP(hipStreamSynchronize(P->st));
   int t0 = 0;  // every instance starts at the same step
@@ -1360,7 +1379,7 @@ int batch_graph(kw_batch* B, int k, const std::string& form, hipGraphExec_t* out
     if (form[i] == '-') continue;
     kw_plan* P = B->plans[i];
     e = hipStreamWaitEvent(P->st, B->fork, 0);
-    for (int s = 0; s < k && rc == KW_OK && e == hipSuccess; ++s) rc = enqueue_step(P, form[i] == 'l');
+    for (int s = 0; s < k && rc == KW_OK && e == hipSuccess; ++s) rc = enqueue_step(P, form[i] == 'l', s, k);
     if (rc == KW_OK && e == hipSuccess) e = hipEventRecord(B->join[i], P->st);
     if (rc == KW_OK && e == hipSuccess) e = hipStreamWaitEvent(B->st, B->join[i], 0);
   }

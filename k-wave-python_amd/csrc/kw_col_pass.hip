@@ -3,20 +3,12 @@
 #include <algorithm>
 #include <mutex>
 
+#include "kw_host.hpp"
 #include "kw_kernels.hpp"
 
 namespace kw {
 
 constexpr int kColDevices = 64;
-
-// Largest pass, in lanes over all its jobs or buffers, that takes the small-grid form
-// (k_col_small): about half the lanes the chip holds at these kernels' registers.  Below,
-// one pass is a chain of latencies (us per step before -> with the form: 128^2 50.9 ->
-// 39.8, 512^2 power law 86.7 -> 72.4, 64^3 power law 116.5 -> 91.2, 64 maps of 128^2 with
-// 133 k lanes a pass 75.8 -> 68.7); above, the narrow tiles' short memory runs cost more
-// than the chain (four 640^2 plus four 512 x 768 lines, 164 k and 197 k lanes a pass: 204
-// either way with the first in this form, 234 with both).
-constexpr int64_t kColSmallLanes = 150000;
 
 // Workgroups of k_col<S, L, OPS> resident on the current device at once (0 if
 // the runtime cannot say).  Queried once per kernel and device.
@@ -65,11 +57,13 @@ static hipError_t col_launch_v(const Geom& g, int nb, const Fields& fl, const Op
   const int ntw = (a.ncols + LW - 1) / LW;
   if ((int64_t)a.nouter * nb * ntw >= 1024 || LW == LS || a.wide) {
     const int gx = col_grid<S, LW, OPS, PV>(a, a.nouter * ntw, nb);
-    hipLaunchKernelGGL((k_col<S, LW, OPS, 1, PV>), dim3(gx, nb), dim3(ColCfg<S, LW, 1, PV>::NT), 0, st, g, fl, ops, inst, a);
+    const ColArgs al = col_blocks(a, gx);
+    hipLaunchKernelGGL((k_col<S, LW, OPS, 1, PV>), dim3(col_gridx(al, ColCfg<S, LW, 1, PV>::NT), nb), dim3(ColCfg<S, LW, 1, PV>::NT), 0, st, g, fl, ops, inst, al);
   } else {
     const int nt = (a.ncols + LS - 1) / LS;
     const int gx = col_grid<S, LS, OPS, PV>(a, a.nouter * nt, nb);
-    hipLaunchKernelGGL((k_col<S, LS, OPS, 1, PV>), dim3(gx, nb), dim3(ColCfg<S, LS, 1, PV>::NT), 0, st, g, fl, ops, inst, a);
+    const ColArgs al = col_blocks(a, gx);
+    hipLaunchKernelGGL((k_col<S, LS, OPS, 1, PV>), dim3(col_gridx(al, ColCfg<S, LS, 1, PV>::NT), nb), dim3(ColCfg<S, LS, 1, PV>::NT), 0, st, g, fl, ops, inst, al);
   }
   return hipGetLastError();
 }
@@ -88,8 +82,9 @@ static hipError_t col_launch_small(const Geom& g, int nb, const Fields& fl, cons
   constexpr int L = col_lsmall2<S>();
   using C = ColCfg<S, L>;
   const int groups = OPS ? a.njob : 1;
-  const dim3 grid(a.nouter * ((a.ncols + L - 1) / L), nb, OPS ? 1 : a.nbuf);
-  hipLaunchKernelGGL((k_col_small<S, L, OPS>), grid, dim3(C::NT * groups), sizeof(float2) * C::LDS * groups, st, g, fl, ops, inst, a);
+  const ColArgs al = col_blocks(a, a.nouter * ((a.ncols + L - 1) / L));
+  const dim3 grid(col_gridx(al, C::NT * groups), nb, OPS ? 1 : a.nbuf);
+  hipLaunchKernelGGL((k_col_small<S, L, OPS>), grid, dim3(C::NT * groups), sizeof(float2) * C::LDS * groups, st, g, fl, ops, inst, al);
   return hipGetLastError();
 }
 
@@ -101,8 +96,7 @@ static hipError_t col_launch(const Geom& g, int nb, const Fields& fl, const Ops&
     if (a.pv && a.small < 2) return col_launch_v<S, LW, OPS, 1>(g, nb, fl, ops, inst, a, st);
   }
   if (a.small && col_small_fits<S, OPS>(a)) {
-    const int64_t lanes = (int64_t)a.nouter * nb * a.ncols * FftShape<S>::TPL * (OPS ? a.njob : a.nbuf);
-    if (a.small == 2 || lanes <= kColSmallLanes) return col_launch_small<S, OPS>(g, nb, fl, ops, inst, a, st);
+    if (a.small == 2 || col_small_lanes(a, S, nb) <= kColSmallLanes) return col_launch_small<S, OPS>(g, nb, fl, ops, inst, a, st);
   }
   return col_launch_v<S, LW, OPS, 0>(g, nb, fl, ops, inst, a, st);
 }

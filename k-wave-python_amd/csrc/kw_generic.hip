@@ -32,6 +32,7 @@
 // rounding of the transforms.
 #include <algorithm>
 
+#include "kw_host.hpp"
 #include "kw_kernels.hpp"
 
 namespace kw {
@@ -385,9 +386,9 @@ __device__ __forceinline__ float2 gswap(float2 a) { return make_float2(a.y, a.x)
 // (tdev), and, for source spectra, instances whose source `which` (-1: p,
 // 0..2: u_i) is not an active spectral (CHAIN) source at this step.
 enum { GF_ALL = -3, GF_ACTIVE = -2 };
-__device__ __forceinline__ bool gen_skip(const int* tdev, const Inst* inst, int b, int which) {
+__device__ __forceinline__ bool gen_skip(const int* tdev, int toff, const Inst* inst, int b, int which) {
   if (which == GF_ALL || !tdev) return false;
-  const int t = gp(tdev)[b];
+  const int t = gp(tdev)[b] + toff;
   const Inst& I = inst[b];
   if (t >= I.nt) return true;
   if (which == GF_ACTIVE) return false;
@@ -465,10 +466,10 @@ __device__ __forceinline__ void gupdate(const Geom& g, int N, int pair0, int P, 
 
 __global__ __launch_bounds__(kGenThreads) void k_gzfwd(Geom g, const float* __restrict__ f, int64_t fs, float2* __restrict__ spec,
                                                        int64_t ss, const float2* __restrict__ twg, GPlan pl, int P, int sp,
-                                                       const int* tdev, const Inst* __restrict__ inst, int which) {
+                                                       const int* tdev, int toff, const Inst* __restrict__ inst, int which) {
   extern __shared__ float2 gsm[];
   const int b = blockIdx.y;
-  if (gen_skip(tdev, inst, b, which)) return;
+  if (gen_skip(tdev, toff, inst, b, which)) return;
   const int N = pl.n;
   const GTw gt(gsm, twg, N);
   const float2* const tw = gsm;
@@ -496,10 +497,10 @@ __global__ __launch_bounds__(kGenThreads) void k_gzfwd(Geom g, const float* __re
 
 __global__ __launch_bounds__(kGenThreads) void k_gzinv(Geom g, const float2* __restrict__ spec, int64_t ss, float* __restrict__ f,
                                                        int64_t fs, const float2* __restrict__ twg, GPlan pl, int P, int sp,
-                                                       float scale, const int* tdev, const Inst* __restrict__ inst, int which) {
+                                                       float scale, const int* tdev, int toff, const Inst* __restrict__ inst, int which) {
   extern __shared__ float2 gsm[];
   const int b = blockIdx.y;
-  if (gen_skip(tdev, inst, b, which)) return;
+  if (gen_skip(tdev, toff, inst, b, which)) return;
   const int N = pl.n;
   const GTw gt(gsm, twg, N);
   const float2* const tw = gsm;
@@ -541,24 +542,24 @@ static int gen_threads(int lines, int n, int64_t groups) {
   return nt;
 }
 static hipError_t gzfwd(const Geom& g, int nb, const float* f, int64_t fs, float2* spec, int64_t ss, const float2* tw,
-                        const int* tdev, const Inst* inst, int which, hipStream_t st) {
+                        const int* tdev, int toff, const Inst* inst, int which, hipStream_t st) {
   const GPlan pl = gplan(g.nz);
   const int npairs = (g.rows + 1) / 2, P = gen_items(g.nz, 1, (int64_t)npairs * nb);
   if (!P) return hipErrorInvalidValue;
   const int blocks = (npairs + P - 1) / P;
   hipLaunchKernelGGL(k_gzfwd, dim3(blocks, nb), dim3(gen_threads(P, g.nz, (int64_t)blocks * nb)), glds_bytes(g.nz, P), st, g, f, fs, spec,
-                     ss, tw, pl, P, gpitch(P), tdev, inst, which);
+                     ss, tw, pl, P, gpitch(P), tdev, toff, inst, which);
   return hipGetLastError();
 }
 
 static hipError_t gzinv(const Geom& g, int nb, const float2* spec, int64_t ss, float* f, int64_t fs, const float2* tw, float scale,
-                        const int* tdev, const Inst* inst, int which, hipStream_t st) {
+                        const int* tdev, int toff, const Inst* inst, int which, hipStream_t st) {
   const GPlan pl = gplan(g.nz);
   const int npairs = (g.rows + 1) / 2, P = gen_items(g.nz, 1, (int64_t)npairs * nb);
   if (!P) return hipErrorInvalidValue;
   const int blocks = (npairs + P - 1) / P;
   hipLaunchKernelGGL(k_gzinv, dim3(blocks, nb), dim3(gen_threads(P, g.nz, (int64_t)blocks * nb)), glds_bytes(g.nz, P), st, g, spec, ss, f,
-                     fs, tw, pl, P, gpitch(P), scale, tdev, inst, which);
+                     fs, tw, pl, P, gpitch(P), scale, tdev, toff, inst, which);
   return hipGetLastError();
 }
 
@@ -600,16 +601,17 @@ __device__ __forceinline__ float2 gjob_op(const XJob& jb, const Ops& ops, const 
 // store, so jobs may write each other's inputs.
 __global__ __launch_bounds__(kGenThreads) void k_gcol(Geom g, Fields fl, Ops ops, const Inst* __restrict__ inst, ColArgs a,
                                                       const float2* __restrict__ twg, GPlan pl, int L, int sp) {
+  if (a.gath && (int)blockIdx.x >= a.gx) return gather_blocks(g, fl, inst, a);
   extern __shared__ float2 gsm[];
   const int b = blockIdx.y;
   const int N = pl.n;
   const GTw gt(gsm, twg, N);
   const float2* const tw = gsm;
-  const int t = fl.tdev ? gp(fl.tdev)[b] : -1, nt = inst[b].nt;
+  const int t = fl.tdev ? step_of(fl, b) : -1, nt = inst[b].nt;
   float2* A = gsm + N;
   float2* B = A + N * sp;
   const int ntile = (a.ncols + L - 1) / L;
-  const int lid = xcd_remap(blockIdx.x, gridDim.x);
+  const int lid = xcd_remap(blockIdx.x, a.gx);
   const int o = lid / ntile, col0 = (lid - o * ntile) * L;
   const int64_t base0 = (int64_t)b * g.nspec + (int64_t)o * a.ostride;
   const int ls = 31 - __clz(L);  // L is a power of two
@@ -681,9 +683,10 @@ __global__ __launch_bounds__(kGenThreads) void k_gcol(Geom g, Fields fl, Ops ops
 // stash spectrum: lines too long for all jobs' buffers in LDS.
 __global__ __launch_bounds__(kGenThreads) void k_gcol_long(Geom g, Fields fl, Ops ops, const Inst* __restrict__ inst, ColArgs a,
                                                            const float2* __restrict__ twg, GPlan pl) {
+  if (a.gath && (int)blockIdx.x >= a.gx) return gather_blocks(g, fl, inst, a);
   extern __shared__ float2 gsm[];
   const int b = blockIdx.y;
-  if (fl.tdev && gp(fl.tdev)[b] >= inst[b].nt) return;
+  if (fl.tdev && step_of(fl, b) >= inst[b].nt) return;
   const int N = pl.n;
   const GTw gt(gsm, twg, N);
   const float2* const tw = gsm;
@@ -721,14 +724,16 @@ hipError_t launch_col_gen(const Geom& g, int nb, const Fields& fl, const Ops& op
   const int L = gen_items(nline, lines, (int64_t)a.nouter * a.ncols * nb);
   if (!L) {
     if (a.mode != 2) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(k_gcol_long, dim3(a.nouter * a.ncols, nb), dim3(kGenThreads), glds_bytes(nline, 1), st, g, fl, ops, inst, a,
+    const ColArgs al = col_blocks(a, a.nouter * a.ncols);
+    hipLaunchKernelGGL(k_gcol_long, dim3(col_gridx(al, kGenThreads), nb), dim3(kGenThreads), glds_bytes(nline, 1), st, g, fl, ops, inst, al,
                        ops.tw[a.axis], pl);
     return hipGetLastError();
   }
   const int ntile = (a.ncols + L - 1) / L, layers = a.mode == 2 ? 1 : a.nbuf;
   const int nt = gen_threads(lines * L, nline, (int64_t)a.nouter * ntile * nb * layers);
-  hipLaunchKernelGGL(k_gcol, dim3(a.nouter * ntile, nb, layers), dim3(nt), glds_bytes(nline, lines * L), st,
-                     g, fl, ops, inst, a, ops.tw[a.axis], pl, L, gpitch(lines * L));
+  const ColArgs al = col_blocks(a, a.nouter * ntile);
+  hipLaunchKernelGGL(k_gcol, dim3(col_gridx(al, nt), nb, layers), dim3(nt), glds_bytes(nline, lines * L), st, g, fl, ops, inst, al,
+                     ops.tw[a.axis], pl, L, gpitch(lines * L));
   return hipGetLastError();
 }
 
@@ -875,7 +880,7 @@ __global__ __launch_bounds__(kGenThreads) void k_gzmom(Geom g, Fields fl, const 
   extern __shared__ float2 gsm[];
   const int b = blockIdx.y, ax = blockIdx.z;
   const Inst& I = inst[b];
-  const int t = gp(fl.tdev)[b];
+  const int t = step_of(fl, b);
   const int N = pl.n;
   const GTw gt(gsm, twg, N);
   const float2* const tw = gsm;
@@ -913,7 +918,7 @@ __global__ __launch_bounds__(kGenThreads) void k_gzmass(Geom g, Fields fl, const
   extern __shared__ float2 gsm[];
   const int b = blockIdx.y;
   const Inst& I = inst[b];
-  const int t = gp(fl.tdev)[b];
+  const int t = step_of(fl, b);
   const int N = pl.n, ND = g.nd;
   const GTw gt(gsm, twg, N);
   const float2* const tw = gsm;
@@ -961,7 +966,7 @@ __global__ __launch_bounds__(kGenThreads) void k_gzeos(Geom g, Fields fl, const 
   extern __shared__ float2 gsm[];
   const int b = blockIdx.y;
   const Inst& I = inst[b];
-  const int t = gp(fl.tdev)[b];
+  const int t = step_of(fl, b);
   const int N = pl.n;
   const GTw gt(gsm, twg, N);
   const float2* const tw = gsm;
@@ -997,7 +1002,7 @@ __global__ __launch_bounds__(kGenThreads) void k_gmomentum(Geom g, Fields fl, co
                                                            const float* __restrict__ gtmp, const float* __restrict__ ctmp) {
   const int b = blockIdx.y;
   const Inst& I = inst[b];
-  const int t = gp(fl.tdev)[b];
+  const int t = step_of(fl, b);
   if (t >= I.nt) return;
   const Src& src = I.srcu[ax];
   const int smode = src_mode_at(src, t);
@@ -1016,7 +1021,7 @@ __global__ __launch_bounds__(kGenThreads) void k_gmass(Geom g, Fields fl, const 
                                                        const float* __restrict__ ctmp, float* aout) {
   const int b = blockIdx.y;
   const Inst& I = inst[b];
-  const int t = gp(fl.tdev)[b];
+  const int t = step_of(fl, b);
   if (t >= I.nt) return;
   const Src& src = I.srcp;
   const int smode = src_mode_at(src, t);
@@ -1037,7 +1042,7 @@ __global__ __launch_bounds__(kGenThreads) void k_geos(Geom g, Fields fl, const I
                                                       const float* __restrict__ av, const float* __restrict__ bv) {
   const int b = blockIdx.y;
   const Inst& I = inst[b];
-  const int t = gp(fl.tdev)[b];
+  const int t = step_of(fl, b);
   if (t >= I.nt) return;
   const int64_t off = (int64_t)b * g.ntot;
   KW_GEN_ELEMENT_LOOP {
@@ -1071,9 +1076,9 @@ __global__ __launch_bounds__(kGenThreads) void k_ginit_u(Geom g, Fields fl, cons
 __global__ __launch_bounds__(kGenThreads) void k_gsrc_scatter(Geom g, Fields fl, const Inst* __restrict__ inst, int which,
                                                               float* __restrict__ out) {
   const int b = blockIdx.y;
-  if (gen_skip(fl.tdev, inst, b, which)) return;
+  if (gen_skip(fl.tdev, fl.toff, inst, b, which)) return;
   const Inst& I = inst[b];
-  const int t = gp(fl.tdev)[b];
+  const int t = step_of(fl, b);
   const Src& s = which < 0 ? I.srcp : I.srcu[which];
   const int64_t off = (int64_t)b * g.ntot;
   KW_GEN_ELEMENT_LOOP {
@@ -1222,12 +1227,12 @@ static dim3 gen_elem_grid(const Geom& g, int nb) {
 // launchers (same contracts as the fused family in kw_launch.hpp)
 // ---------------------------------------------------------------------------
 hipError_t launch_zfwd_gen(const Geom& g, int nb, const float* f, int64_t fs, float2* spec, int64_t ss, const float2* tw, hipStream_t st) {
-  return gzfwd(g, nb, f, fs, spec, ss, tw, nullptr, nullptr, GF_ALL, st);
+  return gzfwd(g, nb, f, fs, spec, ss, tw, nullptr, 0, nullptr, GF_ALL, st);
 }
 
 hipError_t launch_zinv_gen(const Geom& g, int nb, const float2* spec, int64_t ss, float* f, int64_t fs, const float2* tw, float scale,
                            hipStream_t st) {
-  return gzinv(g, nb, spec, ss, f, fs, tw, scale, nullptr, nullptr, GF_ALL, st);
+  return gzinv(g, nb, spec, ss, f, fs, tw, scale, nullptr, 0, nullptr, GF_ALL, st);
 }
 
 // Launch shape of a fused update with `lines` lines per row pair; P = 0: does not fit.
@@ -1259,12 +1264,12 @@ hipError_t launch_momentum_gen(const Geom& g, int nb, const Fields& fl, const In
     return hipGetLastError();
   }
   for (int ax = 0; ax < g.nd; ++ax) {
-    KW_GEN_CHECK(gzinv(g, nb, fl.spec[ax], g.nspec, fl.tmp[0], g.ntot, tw, 1.f, fl.tdev, inst, GF_ACTIVE, st));
+    KW_GEN_CHECK(gzinv(g, nb, fl.spec[ax], g.nspec, fl.tmp[0], g.ntot, tw, 1.f, fl.tdev, fl.toff, inst, GF_ACTIVE, st));
     if (fl.spec[g.nd + 1 + ax])
-      KW_GEN_CHECK(gzinv(g, nb, fl.spec[g.nd + 1 + ax], g.nspec, fl.tmp[3], g.ntot, tw, 1.f, fl.tdev, inst, ax, st));
+      KW_GEN_CHECK(gzinv(g, nb, fl.spec[g.nd + 1 + ax], g.nspec, fl.tmp[3], g.ntot, tw, 1.f, fl.tdev, fl.toff, inst, ax, st));
     hipLaunchKernelGGL(k_gmomentum, gen_elem_grid(g, nb), dim3(kGenThreads), 0, st, g, fl, inst, ax, fl.tmp[0], fl.tmp[3]);
     KW_GEN_CHECK(hipGetLastError());
-    KW_GEN_CHECK(gzfwd(g, nb, fl.u[ax], g.ntot, fl.spec[ax], g.nspec, tw, fl.tdev, inst, GF_ACTIVE, st));
+    KW_GEN_CHECK(gzfwd(g, nb, fl.u[ax], g.ntot, fl.spec[ax], g.nspec, tw, fl.tdev, fl.toff, inst, GF_ACTIVE, st));
   }
   return hipSuccess;
 }
@@ -1275,17 +1280,17 @@ hipError_t launch_mass_gen(const Geom& g, int nb, const Fields& fl, const Inst* 
     hipLaunchKernelGGL(k_gzmass, dim3(f.blocks, nb), dim3(f.nt), f.lds, st, g, fl, inst, tw, flags, f.pl, f.P, f.sp);
     return hipGetLastError();
   }
-  for (int i = 0; i < g.nd; ++i) KW_GEN_CHECK(gzinv(g, nb, fl.spec[i], g.nspec, fl.tmp[i], g.ntot, tw, 1.f, fl.tdev, inst, GF_ACTIVE, st));
-  if (fl.spec[g.nd]) KW_GEN_CHECK(gzinv(g, nb, fl.spec[g.nd], g.nspec, fl.tmp[3], g.ntot, tw, 1.f, fl.tdev, inst, -1, st));
+  for (int i = 0; i < g.nd; ++i) KW_GEN_CHECK(gzinv(g, nb, fl.spec[i], g.nspec, fl.tmp[i], g.ntot, tw, 1.f, fl.tdev, fl.toff, inst, GF_ACTIVE, st));
+  if (fl.spec[g.nd]) KW_GEN_CHECK(gzinv(g, nb, fl.spec[g.nd], g.nspec, fl.tmp[3], g.ntot, tw, 1.f, fl.tdev, fl.toff, inst, -1, st));
   hipLaunchKernelGGL(k_gmass, gen_elem_grid(g, nb), dim3(kGenThreads), 0, st, g, fl, inst, flags, fl.tmp[0], fl.tmp[1], fl.tmp[2],
                      fl.tmp[3], fl.tmp[0]);
   KW_GEN_CHECK(hipGetLastError());
   if (flags & (FLAG_POWERLAW_ABS | FLAG_POWERLAW_DISP)) {
-    if (flags & FLAG_POWERLAW_ABS) KW_GEN_CHECK(gzfwd(g, nb, fl.tmp[0], g.ntot, fl.spec[0], g.nspec, tw, fl.tdev, inst, GF_ACTIVE, st));
-    if (flags & FLAG_POWERLAW_DISP) KW_GEN_CHECK(gzfwd(g, nb, fl.rhot, g.ntot, fl.spec[1], g.nspec, tw, fl.tdev, inst, GF_ACTIVE, st));
+    if (flags & FLAG_POWERLAW_ABS) KW_GEN_CHECK(gzfwd(g, nb, fl.tmp[0], g.ntot, fl.spec[0], g.nspec, tw, fl.tdev, fl.toff, inst, GF_ACTIVE, st));
+    if (flags & FLAG_POWERLAW_DISP) KW_GEN_CHECK(gzfwd(g, nb, fl.rhot, g.ntot, fl.spec[1], g.nspec, tw, fl.tdev, fl.toff, inst, GF_ACTIVE, st));
     return hipSuccess;
   }
-  return gzfwd(g, nb, fl.p, g.ntot, fl.spec[0], g.nspec, tw, fl.tdev, inst, GF_ACTIVE, st);
+  return gzfwd(g, nb, fl.p, g.ntot, fl.spec[0], g.nspec, tw, fl.tdev, fl.toff, inst, GF_ACTIVE, st);
 }
 
 hipError_t launch_eos_gen(const Geom& g, int nb, const Fields& fl, const Inst* inst, const float2* tw, int flags, hipStream_t st) {
@@ -1294,16 +1299,16 @@ hipError_t launch_eos_gen(const Geom& g, int nb, const Fields& fl, const Inst* i
     hipLaunchKernelGGL(k_gzeos, dim3(f.blocks, nb), dim3(f.nt), f.lds, st, g, fl, inst, tw, flags, f.pl, f.P, f.sp);
     return hipGetLastError();
   }
-  if (flags & FLAG_POWERLAW_ABS) KW_GEN_CHECK(gzinv(g, nb, fl.spec[0], g.nspec, fl.tmp[0], g.ntot, tw, 1.f, fl.tdev, inst, GF_ACTIVE, st));
-  if (flags & FLAG_POWERLAW_DISP) KW_GEN_CHECK(gzinv(g, nb, fl.spec[1], g.nspec, fl.tmp[1], g.ntot, tw, 1.f, fl.tdev, inst, GF_ACTIVE, st));
+  if (flags & FLAG_POWERLAW_ABS) KW_GEN_CHECK(gzinv(g, nb, fl.spec[0], g.nspec, fl.tmp[0], g.ntot, tw, 1.f, fl.tdev, fl.toff, inst, GF_ACTIVE, st));
+  if (flags & FLAG_POWERLAW_DISP) KW_GEN_CHECK(gzinv(g, nb, fl.spec[1], g.nspec, fl.tmp[1], g.ntot, tw, 1.f, fl.tdev, fl.toff, inst, GF_ACTIVE, st));
   hipLaunchKernelGGL(k_geos, gen_elem_grid(g, nb), dim3(kGenThreads), 0, st, g, fl, inst, flags, fl.tmp[0], fl.tmp[1]);
   KW_GEN_CHECK(hipGetLastError());
-  return gzfwd(g, nb, fl.p, g.ntot, fl.spec[0], g.nspec, tw, fl.tdev, inst, GF_ACTIVE, st);
+  return gzfwd(g, nb, fl.p, g.ntot, fl.spec[0], g.nspec, tw, fl.tdev, fl.toff, inst, GF_ACTIVE, st);
 }
 
 hipError_t launch_init_u_gen(const Geom& g, int nb, const Fields& fl, const Inst* inst, const float2* tw, hipStream_t st) {
   if (!fl.tmp[0] || !fl.tmp[2]) return hipErrorInvalidValue;
-  for (int ax = 0; ax < g.nd; ++ax) KW_GEN_CHECK(gzinv(g, nb, fl.spec[ax], g.nspec, fl.tmp[ax], g.ntot, tw, 1.f, nullptr, inst, GF_ALL, st));
+  for (int ax = 0; ax < g.nd; ++ax) KW_GEN_CHECK(gzinv(g, nb, fl.spec[ax], g.nspec, fl.tmp[ax], g.ntot, tw, 1.f, nullptr, 0, inst, GF_ALL, st));
   hipLaunchKernelGGL(k_ginit_u, gen_elem_grid(g, nb), dim3(kGenThreads), 0, st, g, fl, inst, fl.tmp[0], fl.tmp[1], fl.tmp[2]);
   return hipGetLastError();
 }
@@ -1313,7 +1318,7 @@ hipError_t launch_src_build_gen(const Geom& g, int nb, const Fields& fl, const I
   const int buf = which < 0 ? g.nd : g.nd + 1 + which;
   hipLaunchKernelGGL(k_gsrc_scatter, gen_elem_grid(g, nb), dim3(kGenThreads), 0, st, g, fl, inst, which, fl.tmp[3]);
   KW_GEN_CHECK(hipGetLastError());
-  return gzfwd(g, nb, fl.tmp[3], g.ntot, fl.spec[buf], g.nspec, tw, fl.tdev, inst, which, st);
+  return gzfwd(g, nb, fl.tmp[3], g.ntot, fl.spec[buf], g.nspec, tw, fl.tdev, fl.toff, inst, which, st);
 }
 
 hipError_t launch_adj_abs1_gen(const Geom& g, int nb, const Fields& fl, const AdjFields& af, const Inst* inst, const float2* tw,
@@ -1321,8 +1326,8 @@ hipError_t launch_adj_abs1_gen(const Geom& g, int nb, const Fields& fl, const Ad
   if (!fl.tmp[0] || !fl.tmp[1]) return hipErrorInvalidValue;
   hipLaunchKernelGGL(k_gadj_abs1, gen_elem_grid(g, nb), dim3(kGenThreads), 0, st, g, af, inst, fl.tmp[0], fl.tmp[1]);
   KW_GEN_CHECK(hipGetLastError());
-  KW_GEN_CHECK(gzfwd(g, nb, fl.tmp[0], g.ntot, fl.spec[0], g.nspec, tw, nullptr, nullptr, GF_ALL, st));
-  if (af.disp) KW_GEN_CHECK(gzfwd(g, nb, fl.tmp[1], g.ntot, fl.spec[1], g.nspec, tw, nullptr, nullptr, GF_ALL, st));
+  KW_GEN_CHECK(gzfwd(g, nb, fl.tmp[0], g.ntot, fl.spec[0], g.nspec, tw, nullptr, 0, nullptr, GF_ALL, st));
+  if (af.disp) KW_GEN_CHECK(gzfwd(g, nb, fl.tmp[1], g.ntot, fl.spec[1], g.nspec, tw, nullptr, 0, nullptr, GF_ALL, st));
   return hipSuccess;
 }
 
@@ -1331,14 +1336,14 @@ hipError_t launch_adj_eos_gen(const Geom& g, int nb, const Fields& fl, const Adj
   if (!fl.tmp[0] || !fl.tmp[2]) return hipErrorInvalidValue;
   if (af.absorb == 2) {  // L1[tau w], L2[eta w] from spectra 0 and 1 (the fractional column passes' outputs)
     if (!af.gl[0] || !af.gl[1]) return hipErrorInvalidValue;
-    KW_GEN_CHECK(gzinv(g, nb, fl.spec[0], g.nspec, af.gl[0], g.ntot, tw, 1.f, nullptr, inst, GF_ALL, st));
-    if (af.disp) KW_GEN_CHECK(gzinv(g, nb, fl.spec[1], g.nspec, af.gl[1], g.ntot, tw, 1.f, nullptr, inst, GF_ALL, st));
+    KW_GEN_CHECK(gzinv(g, nb, fl.spec[0], g.nspec, af.gl[0], g.ntot, tw, 1.f, nullptr, 0, inst, GF_ALL, st));
+    if (af.disp) KW_GEN_CHECK(gzinv(g, nb, fl.spec[1], g.nspec, af.gl[1], g.ntot, tw, 1.f, nullptr, 0, inst, GF_ALL, st));
   }
   hipLaunchKernelGGL(k_gadj_eos, gen_elem_grid(g, nb), dim3(kGenThreads), 0, st, g, af, inst, t, af.gl[0], af.gl[1], fl.tmp[0],
                      fl.tmp[1], fl.tmp[2]);
   KW_GEN_CHECK(hipGetLastError());
   for (int i = 0; i < g.nd; ++i)
-    KW_GEN_CHECK(gzfwd(g, nb, fl.tmp[i], g.ntot, fl.spec[i], g.nspec, tw, nullptr, nullptr, GF_ALL, st));
+    KW_GEN_CHECK(gzfwd(g, nb, fl.tmp[i], g.ntot, fl.spec[i], g.nspec, tw, nullptr, 0, nullptr, GF_ALL, st));
   return hipSuccess;
 }
 
@@ -1346,10 +1351,10 @@ hipError_t launch_adj_mom_gen(const Geom& g, int nb, const Fields& fl, const Adj
                               hipStream_t st) {
   if (!fl.tmp[0] || !fl.tmp[1]) return hipErrorInvalidValue;
   for (int ax = 0; ax < g.nd; ++ax) {
-    KW_GEN_CHECK(gzinv(g, nb, fl.spec[ax], g.nspec, fl.tmp[0], g.ntot, tw, 1.f, nullptr, inst, GF_ALL, st));
+    KW_GEN_CHECK(gzinv(g, nb, fl.spec[ax], g.nspec, fl.tmp[0], g.ntot, tw, 1.f, nullptr, 0, inst, GF_ALL, st));
     hipLaunchKernelGGL(k_gadj_mom, gen_elem_grid(g, nb), dim3(kGenThreads), 0, st, g, af, inst, t, ax, fl.tmp[0], fl.tmp[1]);
     KW_GEN_CHECK(hipGetLastError());
-    KW_GEN_CHECK(gzfwd(g, nb, fl.tmp[1], g.ntot, fl.spec[ax], g.nspec, tw, nullptr, nullptr, GF_ALL, st));
+    KW_GEN_CHECK(gzfwd(g, nb, fl.tmp[1], g.ntot, fl.spec[ax], g.nspec, tw, nullptr, 0, nullptr, GF_ALL, st));
   }
   return hipSuccess;
 }
@@ -1358,7 +1363,7 @@ hipError_t launch_adj_sum_gen(const Geom& g, int nb, const Fields& fl, const Adj
                               hipStream_t st) {
   if (!fl.tmp[0] || !fl.tmp[2]) return hipErrorInvalidValue;
   for (int i = 0; i < g.nd; ++i)
-    KW_GEN_CHECK(gzinv(g, nb, fl.spec[i], g.nspec, fl.tmp[i], g.ntot, tw, 1.f, nullptr, inst, GF_ALL, st));
+    KW_GEN_CHECK(gzinv(g, nb, fl.spec[i], g.nspec, fl.tmp[i], g.ntot, tw, 1.f, nullptr, 0, inst, GF_ALL, st));
   hipLaunchKernelGGL(k_gadj_sum, gen_elem_grid(g, nb), dim3(kGenThreads), 0, st, g, af, fl.tmp[0], fl.tmp[1], fl.tmp[2]);
   return hipGetLastError();
 }

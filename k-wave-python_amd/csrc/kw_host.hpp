@@ -10,6 +10,7 @@
 #include <string>
 #include <vector>
 
+#include "kw_fft.hpp"
 #include "kw_types.hpp"
 
 namespace kw {
@@ -66,6 +67,26 @@ inline Geom make_geom(int nd, const int* n) {
   g.small = 1;
   return g;
 }
+
+// Largest pass, in lanes over all its jobs or buffers, that takes the small-grid form
+// (k_col_small): about half the lanes the chip holds at these kernels' registers.  Below,
+// one pass is a chain of latencies (us per step before -> with the form: 128^2 50.9 ->
+// 39.8, 512^2 power law 86.7 -> 72.4, 64^3 power law 116.5 -> 91.2, 64 maps of 128^2 with
+// 133 k lanes a pass 75.8 -> 68.7); above, the narrow tiles' short memory runs cost more
+// than the chain (four 640^2 plus four 512 x 768 lines, 164 k and 197 k lanes a pass: 204
+// either way with the first in this form, 234 with both).
+constexpr int64_t kColSmallLanes = 150000;
+// lanes of a column pass over a compiled line length
+inline int64_t col_small_lanes(const ColArgs& a, int nline, int nb) {
+  return (int64_t)a.nouter * nb * a.ncols * (nline / plan_elems(nline)) * (a.mode == 2 ? a.njob : a.nbuf);
+}
+// a column pass of gx workgroups an instance, and its grid with the gathering ones
+inline ColArgs col_blocks(const ColArgs& a, int gx) {
+  ColArgs r = a;
+  r.gx = gx;
+  return r;
+}
+inline unsigned col_gridx(const ColArgs& a, int threads) { return (unsigned)(a.gx + (a.gath + threads - 1) / threads); }
 
 inline ColArgs col_args(const Geom& g, int axis, int mode) {
   ColArgs a{};

@@ -75,6 +75,51 @@ __device__ __forceinline__ void st2(KW_AS1 float2* p, int64_t i, float2 v) {
 
 __device__ __forceinline__ float ld(const float* p, int64_t i, int s) { return gp(p)[i * s]; }
 
+// step an instance is at
+__device__ __forceinline__ int step_of(const Fields& fl, int b) { return gp(fl.tdev)[b] + fl.toff; }
+
+// Record sensor s of instance b at step t: interpolated pressure and velocities, running
+// maximum, minimum and sum of squares.
+__device__ __forceinline__ void gather_point(const Geom& g, const Fields& fl, const Inst& I, int b, int t, int s) {
+  if (I.sens_kind == 0 || t >= I.nt || t < I.rec_start || s >= I.nsens) return;
+  const int64_t off = b * g.ntot;
+  const int64_t row = (int64_t)(t - I.rec_start) * I.nsens + s;
+  auto sample = [&](const float* f) {
+    float acc = 0.f;
+    for (int c = 0; c < I.ncorner; ++c) {
+      const int64_t ii = I.sidx[(int64_t)s * I.ncorner + c];
+      const float w = I.sens_kind == 2 ? I.sw[(int64_t)s * I.ncorner + c] : 1.f;
+      acc += w * f[off + ii];
+    }
+    return acc;
+  };
+  if (I.rec_p || I.agg_p) {
+    const float v = sample(fl.p);
+    if (I.rec_p) I.rec_p[row] = v;
+    if (I.agg_p) {
+      float* a = I.agg_p;
+      if (t == I.rec_start) { a[s] = v; a[I.nsens + s] = v; a[2 * I.nsens + s] = v * v; }
+      else { a[s] = fmaxf(a[s], v); a[I.nsens + s] = fminf(a[I.nsens + s], v); a[2 * I.nsens + s] += v * v; }
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < 3; ++i) {
+    if (i >= g.nd) continue;
+    if (I.rec_u[i]) I.rec_u[i][row] = sample(fl.u[i]);
+    if (I.rec_uc[i]) I.rec_uc[i][row] = sample(fl.uc[i]);
+  }
+}
+// The workgroups a column pass has beyond its own (ColArgs::gath): the sensors of the step
+// before, whose fields nothing changes before the next update.  A kernel of its own would
+// add its launch and one chain of latencies, 4 to 5 us, to every step (with the counter
+// advanced once a block as well, us per step: 128^2 30.0 -> 25.7, 512^2 power law 51.3 ->
+// 48.4, 64 maps of 128^2 58.5 -> 54.7).
+__device__ __forceinline__ void gather_blocks(const Geom& g, const Fields& fl, const Inst* inst, const ColArgs& a) {
+  if (blockIdx.z) return;
+  const int b = blockIdx.y;
+  gather_point(g, fl, inst[b], b, step_of(fl, b) - 1, ((int)blockIdx.x - a.gx) * (int)blockDim.x + (int)threadIdx.x);
+}
+
 // absorption / dispersion coefficient at idx given c0^2 there
 __device__ __forceinline__ float tau_at(const Inst& I, int64_t idx, float c2) {
   return I.tau ? ld(I.tau, idx, I.tau_s) : I.tau_c * exp2f(I.ym1h * log2f(c2));
@@ -450,7 +495,7 @@ __global__ __launch_bounds__(ZCfg<N>::NT) KW_WPE(N, KW_WPE_MOM) void k_momentum(
   const int ax = blockIdx.z;
   const bool zax = ax == g.nd - 1;
   KW_ZPASS_EARLY(zax ? inst[blockIdx.y].pmlsg[ax] : nullptr)
-  const int t = gp(fl.tdev)[b];
+  const int t = step_of(fl, b);
   KW_ROWS_CLAMPED
   float2* sp = fl.spec[ax] + b * g.nspec;
   const auto u = gw(fl.u[ax] + b * g.ntot);
@@ -519,7 +564,7 @@ __global__ __launch_bounds__(ZCfg<N>::NT) KW_WPE(N, KW_WPE_MOM) void k_momentum(
 template <int N, int ND, bool SREG, bool CAP>
 __global__ __launch_bounds__(ZCfg<N>::NT) KW_WPE(N, KW_WPE_MASS) void k_mass(Geom g, Fields fl, const Inst* __restrict__ inst, const float2* __restrict__ tw_g, int flags) {
   KW_ZPASS_EARLY(inst[blockIdx.y].pml[ND - 1])
-  const int t = gp(fl.tdev)[b];
+  const int t = step_of(fl, b);
   KW_ROWS_CLAMPED
   const int64_t off = b * g.ntot;
   const Src& src = I.srcp;
@@ -722,7 +767,7 @@ __global__ __launch_bounds__(ZCfg<N>::NT) KW_WPE(N, KW_WPE_MASS) void k_mass(Geo
 template <int N>
 __global__ __launch_bounds__(ZCfg<N>::NT) KW_WPE(N, KW_WPE_EOS) void k_eos(Geom g, Fields fl, const Inst* __restrict__ inst, const float2* __restrict__ tw_g, int flags) {
   KW_ZPASS_EARLY((const float*)nullptr)
-  const int t = gp(fl.tdev)[b];
+  const int t = step_of(fl, b);
   KW_ROWS_CLAMPED
   const int64_t off = b * g.ntot;
   const auto rhot = gw(fl.rhot + off);
@@ -832,7 +877,7 @@ template <int N, bool NAR>
 __global__ __launch_bounds__((ZCfg<N, NAR>::NT)) void k_src_build(Geom g, Fields fl, const Inst* __restrict__ inst, const float2* __restrict__ tw_g, int which) {
   KW_ZPASS_PROLOGUE_AS(ZCfg<N, NAR>)
   const Inst& I = inst[b];
-  const int t = gp(fl.tdev)[b];
+  const int t = step_of(fl, b);
   const Src& s = which < 0 ? I.srcp : I.srcu[which];
   if (t >= I.nt || s.mode != SRC_CHAIN || t >= s.len) return;
   const auto sp = gw(fl.spec[s.chain_buf] + b * g.nspec);
@@ -979,13 +1024,14 @@ constexpr int col_lops() { return col_lbig<N>() / 2 < 1 ? 1 : col_lbig<N>() / 2;
 
 template <int N, int L, bool OPS, int EM = 1, int PV = 0>
 __global__ __launch_bounds__((ColCfg<N, L, EM, PV>::NT)) KW_WPE(N, (OPS ? KW_WPE_COLOPS : KW_WPE_COL)) void k_col(Geom g, Fields fl, Ops ops, const Inst* __restrict__ inst, ColArgs a) {
+  if (a.gath && (int)blockIdx.x >= a.gx) return gather_blocks(g, fl, inst, a);
   using C = ColCfg<N, L, EM, PV>;
   __shared__ float2 lds[C::LDS];
   __shared__ float2 twl[stage_tw_size<N, PV>()];
   const typename C::Idx idx{};
   const int tid = threadIdx.x;
   const int b = blockIdx.y;
-  if (fl.tdev && gp(fl.tdev)[b] >= inst[b].nt) return;
+  if (fl.tdev && step_of(fl, b) >= inst[b].nt) return;
   {
     float2 twr[stage_tw_loads<N, PV>(C::NT)];
     load_stage_tw<N, PV, C::NT>(twr, ops.tw[a.axis], tid);
@@ -993,7 +1039,7 @@ __global__ __launch_bounds__((ColCfg<N, L, EM, PV>::NT)) KW_WPE(N, (OPS ? KW_WPE
   }
   __syncthreads();
   const int ntile = (a.ncols + L - 1) / L;
-  const int lid = xcd_remap(blockIdx.x, gridDim.x);
+  const int lid = xcd_remap(blockIdx.x, a.gx);
   const int c = tid % L, j0 = tid / L;
   const float2* tw = twl;
   const int ntiles = a.nouter * ntile;
@@ -1020,8 +1066,8 @@ __global__ __launch_bounds__((ColCfg<N, L, EM, PV>::NT)) KW_WPE(N, (OPS ? KW_WPE
 #pragma unroll
       for (int m = 0; m < C::E; ++m) nx[m] = ld2(bp, bt + m * step);
     }
-    for (int lt = lid; lt < ntiles; lt += (int)gridDim.x) {
-      const int ltn = lt + (int)gridDim.x;
+    for (int lt = lid; lt < ntiles; lt += a.gx) {
+      const int ltn = lt + a.gx;
       bool vn = false;
       const int64_t bn = tile_base(min(ltn, ntiles - 1), vn);
       for (int q = 0; q < a.nbuf; ++q) {
@@ -1081,7 +1127,7 @@ __global__ __launch_bounds__((ColCfg<N, L, EM, PV>::NT)) KW_WPE(N, (OPS ? KW_WPE
   constexpr bool PRE = C::E <= 8;
   float2 nx[PRE ? C::E : 1];
   bool next_loaded = false;  // nx holds this tile's first input
-  for (int lt = lid; lt < ntiles; lt += (int)gridDim.x) {
+  for (int lt = lid; lt < ntiles; lt += a.gx) {
     const int o = lt / ntile, tile = lt % ntile;
     const int col = tile * L + c;
     bool valid = false;
@@ -1138,9 +1184,9 @@ __global__ __launch_bounds__((ColCfg<N, L, EM, PV>::NT)) KW_WPE(N, (OPS ? KW_WPE
             bool clobbered = false;
             for (int i = j; i < k; ++i) clobbered |= a.job[i].out == a.job[k].in;
             if (!clobbered) from = pre_in = a.job[k].in;
-          } else if (lt + (int)gridDim.x < ntiles) {
+          } else if (lt + a.gx < ntiles) {
             bool vn;
-            nbase = tile_base(lt + (int)gridDim.x, vn);
+            nbase = tile_base(lt + a.gx, vn);
             from = a.job[0].in;
             next_loaded = true;
           }
@@ -1220,6 +1266,7 @@ constexpr int col_lsmall2() { return clampi(64 / FftShape<N>::TPL, KW_COL_SMALL_
 
 template <int N, int L, bool OPS>
 __global__ __launch_bounds__((ColCfg<N, L>::NT * (OPS ? kColSmallJobs : 1))) void k_col_small(Geom g, Fields fl, Ops ops, const Inst* __restrict__ inst, ColArgs a) {
+  if (a.gath && (int)blockIdx.x >= a.gx) return gather_blocks(g, fl, inst, a);
   using C = ColCfg<N, L>;
   constexpr bool WS = C::NT == 64;
   extern __shared__ float2 lds_all[];
@@ -1230,7 +1277,7 @@ __global__ __launch_bounds__((ColCfg<N, L>::NT * (OPS ? kColSmallJobs : 1))) voi
   const int b = blockIdx.y;
   float2* const lds = lds_all + grp * C::LDS;
   const int ntile = (a.ncols + L - 1) / L;
-  const int lid = xcd_remap(blockIdx.x, gridDim.x);
+  const int lid = xcd_remap(blockIdx.x, a.gx);
   const int o = lid / ntile, tile = lid % ntile;
   const int c = tid % L, j0 = tid / L;
   const int col = tile * L + c;
@@ -1269,7 +1316,7 @@ __global__ __launch_bounds__((ColCfg<N, L>::NT * (OPS ? kColSmallJobs : 1))) voi
     kyz2 = ky * ky;
     if (g.nd == 3) { const float kz = gp(ops.k[2])[valid ? col : 0]; kyz2 = fmaf(kz, kz, kyz2); }
   }
-  if (fl.tdev && gp(fl.tdev)[b] >= inst[b].nt) return;
+  if (fl.tdev && step_of(fl, b) >= inst[b].nt) return;
   if (grp == 0) put_stage_tw<N, 0, C::NT>(twr, twl, tid);
   __syncthreads();
   if constexpr (!OPS) {
@@ -1345,7 +1392,7 @@ __global__ __launch_bounds__((ZCfg<N, true>::NT)) void k_momentum_small(Geom g, 
   float2 As[C::IT], Bs[C::IT];
   pair_load<C>(As, Bs, sp, row0, rows, g.nhp, tid);
   load_stage_tw<N, C::PV, G * C::NT>(twr, tw_g, threadIdx.x);
-  const int t = gp(fl.tdev)[b];
+  const int t = step_of(fl, b);
   KW_ROWS_CLAMPED
   const auto u = gw(fl.u[ax] + b * g.ntot);
   const Src& src = I.srcu[ax];
@@ -1410,7 +1457,7 @@ __global__ __launch_bounds__((ZCfg<N, true>::NT * ND)) void k_mass_small(Geom g,
   float2 As[C::IT], Bs[C::IT];
   pair_load<C>(As, Bs, fl.spec[grp] + b * g.nspec, row0, rows, g.nhp, tid);
   load_stage_tw<N, C::PV, G * C::NT>(twr, tw_g, threadIdx.x);
-  const int t = gp(fl.tdev)[b];
+  const int t = step_of(fl, b);
   KW_ROWS_CLAMPED
   const int64_t off = b * g.ntot;
   const Src& src = I.srcp;
@@ -1559,7 +1606,7 @@ __global__ __launch_bounds__((ZCfg<N, true>::NT * 2)) void k_eos_small(Geom g, F
   float2 As[C::IT], Bs[C::IT];
   pair_load<C>(As, Bs, fl.spec[grp] + b * g.nspec, row0, rows, g.nhp, tid);
   load_stage_tw<N, C::PV, G * C::NT>(twr, tw_g, threadIdx.x);
-  const int t = gp(fl.tdev)[b];
+  const int t = step_of(fl, b);
   KW_ROWS_CLAMPED
   const int64_t off = b * g.ntot;
   float2 rtv[C::E], c2v[C::E], r0v[C::E], bav[C::E], co[C::E];

@@ -36,7 +36,9 @@ hipError_t launch_init_u(const Geom& g, int nb, const Fields& fl, const Inst* in
 hipError_t launch_src_build(const Geom& g, int nb, const Fields& fl, const Inst* inst, const float2* tw, int which, hipStream_t st);
 hipError_t launch_col(const Geom& g, int nb, const Fields& fl, const Ops& ops, const Inst* inst, const ColArgs& a, int nline, hipStream_t st);
 hipError_t launch_gather(const Geom& g, int nb, int max_sens, const Fields& fl, const Inst* inst, hipStream_t st);
-hipError_t launch_tick(const Fields& fl, const Inst* inst, int nb, hipStream_t st);
+// advance the step counters by n (not beyond an instance's last step); with the sensors of the step gathered first
+hipError_t launch_tick(const Fields& fl, const Inst* inst, int nb, int n, hipStream_t st);
+hipError_t launch_gather_tick(const Geom& g, int nb, int max_sens, const Fields& fl, const Inst* inst, int n, hipStream_t st);
 hipError_t launch_fill(float* p, int64_t n, float v, hipStream_t st);
 hipError_t launch_setint(int* p, int n, int v, hipStream_t st);
 // surrogate (kw_fno.hip)

@@ -10,40 +10,23 @@ namespace kw {
 // ---------------------------------------------------------------------------
 __global__ void k_gather(Geom g, Fields fl, const Inst* __restrict__ inst) {
   const int b = blockIdx.y;
-  const Inst& I = inst[b];
-  const int t = fl.tdev[b];
-  if (I.sens_kind == 0 || t >= I.nt || t < I.rec_start) return;
-  const int s = blockIdx.x * blockDim.x + threadIdx.x;
-  if (s >= I.nsens) return;
-  const int64_t off = b * g.ntot;
-  const int64_t row = (int64_t)(t - I.rec_start) * I.nsens + s;
-  auto sample = [&](const float* f) {
-    float acc = 0.f;
-    for (int c = 0; c < I.ncorner; ++c) {
-      const int64_t ii = I.sidx[(int64_t)s * I.ncorner + c];
-      const float w = I.sens_kind == 2 ? I.sw[(int64_t)s * I.ncorner + c] : 1.f;
-      acc += w * f[off + ii];
-    }
-    return acc;
-  };
-  if (I.rec_p || I.agg_p) {
-    const float v = sample(fl.p);
-    if (I.rec_p) I.rec_p[row] = v;
-    if (I.agg_p) {
-      float* a = I.agg_p;
-      if (t == I.rec_start) { a[s] = v; a[I.nsens + s] = v; a[2 * I.nsens + s] = v * v; }
-      else { a[s] = fmaxf(a[s], v); a[I.nsens + s] = fminf(a[I.nsens + s], v); a[2 * I.nsens + s] += v * v; }
-    }
-  }
-  for (int i = 0; i < g.nd; ++i) {
-    if (I.rec_u[i]) I.rec_u[i][row] = sample(fl.u[i]);
-    if (I.rec_uc[i]) I.rec_uc[i][row] = sample(fl.uc[i]);
-  }
+  gather_point(g, fl, inst[b], b, step_of(fl, b), blockIdx.x * blockDim.x + threadIdx.x);
 }
 
-__global__ void k_tick(Fields fl, const Inst* __restrict__ inst, int nb) {
-  for (int b = threadIdx.x; b < nb; b += blockDim.x)
-    if (fl.tdev[b] < inst[b].nt) fl.tdev[b] += 1;
+__global__ void k_tick(Fields fl, const Inst* __restrict__ inst, int nb, int n) {
+  for (int b = threadIdx.x; b < nb; b += blockDim.x) fl.tdev[b] = min(fl.tdev[b] + n, max(fl.tdev[b], inst[b].nt));
+}
+
+// both, for instances with few sensors: one workgroup an instance, which reads the
+// counter before it advances it
+__global__ __launch_bounds__(256) void k_gather_tick(Geom g, Fields fl, const Inst* __restrict__ inst, int n) {
+  const int b = blockIdx.x;
+  const Inst& I = inst[b];
+  const int t0 = fl.tdev[b], t = t0 + fl.toff;
+  if (t < I.nt)
+    for (int s = threadIdx.x; s < I.nsens; s += blockDim.x) gather_point(g, fl, I, b, t, s);
+  __syncthreads();
+  if (threadIdx.x == 0) fl.tdev[b] = min(t0 + n, max(t0, I.nt));
 }
 
 __global__ void k_fill(float* __restrict__ p, int64_t n, float v) {
@@ -146,8 +129,18 @@ hipError_t launch_gather(const Geom& g, int nb, int max_sens, const Fields& fl, 
   return hipGetLastError();
 }
 
-hipError_t launch_tick(const Fields& fl, const Inst* inst, int nb, hipStream_t st) {
-  hipLaunchKernelGGL(k_tick, dim3(1), dim3(256), 0, st, fl, inst, nb);
+hipError_t launch_tick(const Fields& fl, const Inst* inst, int nb, int n, hipStream_t st) {
+  hipLaunchKernelGGL(k_tick, dim3(1), dim3(256), 0, st, fl, inst, nb, n);
+  return hipGetLastError();
+}
+
+// one launch for both up to 4096 sensors (16 a thread)
+hipError_t launch_gather_tick(const Geom& g, int nb, int max_sens, const Fields& fl, const Inst* inst, int n, hipStream_t st) {
+  if (max_sens > 4096) {
+    const hipError_t e = launch_gather(g, nb, max_sens, fl, inst, st);
+    return e != hipSuccess ? e : launch_tick(fl, inst, nb, n, st);
+  }
+  hipLaunchKernelGGL(k_gather_tick, dim3(nb), dim3(256), 0, st, g, fl, inst, n);
   return hipGetLastError();
 }
 

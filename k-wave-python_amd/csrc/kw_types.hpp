@@ -107,6 +107,8 @@ struct ColArgs {
   int persist;      // passes whose workgroups may loop over tiles: bit 0 with jobs, bit 1 FFT-only
   int grid;         // > 0: workgroups per instance when looping (tests of the loop on small grids)
   int small;        // small-grid form of the pass: 0 never, 1 by the size rule (kw_col_pass.hip), 2 always where it applies
+  int gath;         // > 0: the pass also gathers the sensors (at most gath points an instance) of the step before, in workgroups of its own
+  int gx;           // workgroups of the pass itself per instance (set by the launcher)
   int pv;           // radix-plan variant of the transform (lengths with a factor 5 or 7; chosen per plan by timing)
 };
 
@@ -118,6 +120,7 @@ struct Fields {
   float2* spec[kMaxBufs];
   float* uc[3];     // velocity on the pressure grid (only when it is recorded)
   int* tdev;        // per-instance step counter
+  int toff;         // steps since the counter was last advanced (a captured block advances it once, at its end)
   // generic-length family only (kw_generic.hip): real temporaries of the unfused
   // contiguous-axis updates, and the stash of a column pass's forward transform
   float* tmp[4];

@@ -69,3 +69,31 @@ def test_small_grid_forms_give_the_same_bits(shape, absorb, bona, monkeypatch):
     for form in ("1", "2"):
         for k, v in run(form).items():
             assert np.array_equal(v, large[k]), (form, k)
+
+
+@pytest.mark.parametrize("shape", [(70, 66), (128, 64), (20, 18, 16), (32, 16, 24)])
+@pytest.mark.parametrize("sensor", ["all", "few"])
+def test_records_do_not_depend_on_how_steps_are_grouped(shape, sensor, monkeypatch):
+    """Steps run in captured blocks gather a step's sensors in the next step's first column
+    pass; run(), step() and the graph-free path record the same bits, with few sensors (one
+    workgroup gathers and advances the counter) and with more than 4096 (two launches)."""
+    from kwave_amd.solvers.kspace_solver import Simulation
+
+    kg, med, src, sen = _case(shape, (0.5, 1.3), None)
+    if sensor == "all":
+        sen.mask = np.ones(shape, dtype=bool)
+    sen.record = ["p", "p_max", "u", "u_staggered", "p_final"]
+    sen.record_start_index = 3
+
+    def make():
+        return Simulation(kg, med, copy.deepcopy(src), sen, pml_size=(3,) * len(shape), pml_alpha=(2.0,) * len(shape))
+
+    blocks = make().run()
+    sim = make()
+    sim.setup()
+    while sim.t < sim.Nt:
+        sim.step()
+    monkeypatch.setenv("KW_NO_GRAPH", "1")
+    for other in (sim.run(), make().run()):
+        for k, v in blocks.items():
+            assert np.array_equal(v, other[k]), k
