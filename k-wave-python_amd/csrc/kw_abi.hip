@@ -102,6 +102,7 @@ struct kw_plan {
   bool lean = true;      // use the lean step form once filtered sources have ended
   bool graphs = true;
   bool skip_gather = false;  // replayed steps of the reverse sweep do not record
+  float *p_out = nullptr, *rhot_out = nullptr;  // where the step's p and density sum go (reverse sweep; null: in place)
   int col_tile[2] = {0, 0};  // tile variant of the FFT-only and the spectral-job column passes
   int col_pv[2] = {0, 0};    // radix-plan variant of those passes (lengths with a factor 5 or 7)
   bool tuned = false;
@@ -329,6 +330,9 @@ int enqueue_step(kw_plan* P, bool lean = false, int j = 0, int k = 1) {
   for (int i = 0; i < D; ++i)
     if (P->rec_uc[i])
       KW_TLAUNCH(KK_SRC, 0.0, launch_zinv(g, P->nb, P->fl.spec[2 * D + 1 + i], g.nspec, P->fl.uc[i], g.ntot, twz, 1.f, P->st));
+  // (the sensors of the step before were read by its first column pass)
+  if (P->p_out) P->fl.p = P->p_out;
+  if (P->rhot_out) P->fl.rhot = P->rhot_out;
   KW_TLAUNCH(KK_MASS, zbytes_mass(P), launch_mass(g, P->nb, P->fl, P->d_inst, twz, P->flags, P->st, (P->chain_p || P->pattern_p) && !lean));
   if (P->flags & (KW_POWERLAW_ABS | KW_POWERLAW_DISP)) {
     jobs.clear();
@@ -464,6 +468,7 @@ int kw_plan_create(const kw_plan_desc* d, kw_plan** out) {
   // sum of the split densities: EOS input (power law) and nonlinear factor of the next step
   if (P->flags & (KW_POWERLAW_ABS | KW_POWERLAW_DISP | KW_NONLINEAR))
     if ((rc = P->mem.alloc(&P->fl.rhot, nf))) return cleanup(rc);
+    P->fl.rhoi = P->fl.rhot;
   if ((rc = ensure_spec(P, d->ndim - 1))) return cleanup(rc);
   // generic-length family (kw_generic.hip): real temporaries for the unfused
   // contiguous-axis updates, a stash spectrum for column passes with jobs
@@ -1128,9 +1133,9 @@ int kw_plan_adjoint_c(kw_plan* P, const float* adj, int ckpt, float* grad_c) {
   const bool nonlin = (P->flags & KW_NONLINEAR) != 0;
   const int nstate = 2 * D + 1 + (nonlin ? 1 : 0);  // p, u_i, rho_i (, sum of rho_i)
   DevBuf tmp;                    // freed when the call returns
-  float *ck, *pbuf, *Zbuf, *dadj;
+  float *ck = nullptr, *pbuf, *Zbuf, *dadj;
   AdjFields af{};
-  if ((rc = tmp.alloc(&ck, (size_t)nck * nstate * nf)) || (rc = tmp.alloc(&pbuf, (size_t)std::min(ckpt, nt) * nf)) ||
+  if ((nck > 1 && (rc = tmp.alloc(&ck, (size_t)(nck - 1) * nstate * nf))) || (rc = tmp.alloc(&pbuf, (size_t)std::min(ckpt, nt) * nf)) ||
       (rc = tmp.alloc(&af.pb, (size_t)nf)) || (rc = tmp.alloc(&af.cb, (size_t)nf)) || (rc = tmp.alloc(&af.R, (size_t)nf)) ||
       (rc = tmp.alloc(&Zbuf, (size_t)nf)) || (rc = tmp.upload(&dadj, adj, (size_t)nb * nrec * I0.nsens)))
     return rc;
@@ -1154,34 +1159,70 @@ int kw_plan_adjoint_c(kw_plan* P, const float* adj, int ckpt, float* grad_c) {
   if (af.disp && (rc = tmp.alloc(&bbuf, (size_t)std::min(ckpt, nt) * nf))) return rc;
   // generic-length contiguous axis with the power law: L1[tau w] and L2[eta w] on the grid
   if (generic_z(g) && af.absorb == 2 && ((rc = tmp.alloc(&af.gl[0], (size_t)nf)) || (rc = tmp.alloc(&af.gl[1], (size_t)nf)))) return rc;
-  // B/A: the replay keeps the density sum before and after every step (ckpt + 1 slots)
-  // and each step's per-axis Dop_i u_i
+  // B/A: the replay keeps the density sum after every step and each step's per-axis Dop_i u_i
   float *sbuf = nullptr, *dbuf = nullptr;
   af.nonlin = nonlin ? 1 : 0;
-  if (nonlin && ((rc = tmp.alloc(&sbuf, (size_t)(std::min(ckpt, nt) + 1) * nf)) ||
+  if (nonlin && ((rc = tmp.alloc(&sbuf, (size_t)std::min(ckpt, nt) * nf)) ||
                  (rc = tmp.alloc(&dbuf, (size_t)std::min(ckpt, nt) * D * nf))))
     return rc;
   af.adj = dadj;
   af.nrec = nrec;
   af.nsens = I0.nsens;
-  std::vector<float*> state = {P->fl.p};
+  float *const p_state = P->fl.p, *const rhot_state = P->fl.rhot;
+  std::vector<float*> state = {p_state};
   for (int i = 0; i < D; ++i) state.push_back(P->fl.u[i]);
   for (int i = 0; i < D; ++i) state.push_back(P->fl.rho[i]);
-  if (nonlin) state.push_back(P->fl.rhot);
+  if (nonlin) state.push_back(rhot_state);
   auto copy_state = [&](int k, bool save) -> int {
+    CopyList c{};
+    c.count = nstate;
     for (int s = 0; s < nstate; ++s) {
       float* slot = ck + ((int64_t)k * nstate + s) * nf;
-      KW_HIP(hipMemcpyAsync(save ? slot : state[s], save ? state[s] : slot, sizeof(float) * nf, hipMemcpyDeviceToDevice, P->st));
+      c.src[s] = save ? state[s] : slot;
+      c.dst[s] = save ? slot : state[s];
     }
+    KW_LAUNCH(launch_copies(c, nf, P->st));
     return KW_OK;
   };
-  // forward pass: records the traces, keeps the state before every ckpt-th step
+  int* const tdev = P->fl.tdev;
+  auto restore_plan = [&] {  // the plan's own buffers, whatever ended the sweep
+    P->fl.p = p_state;
+    P->fl.rhot = rhot_state;
+    P->fl.rhoi = rhot_state;
+    P->fl.adjA = P->fl.adjB = P->fl.adjD = nullptr;
+    P->fl.tdev = tdev;
+    P->p_out = P->rhot_out = nullptr;
+    P->skip_gather = false;
+  };
+  const int64_t qend = P->lean ? source_end(P) : -1;
+  // The steps of segment seg from the state before it.  keep: p, the density sum and the
+  // absorption and divergence operands of every step go straight to their slots, so the
+  // next step reads the sum from there and nothing is copied.
+  auto run_segment = [&](int seg, bool keep) -> int {
+    const int t0 = tb + seg * ckpt, t1 = std::min(nt, t0 + ckpt);
+    int r = KW_OK;
+    for (int t = t0; t < t1 && r == KW_OK; ++t) {
+      if (keep) {
+        const int64_t k = t - t0;
+        P->fl.adjA = abuf ? abuf + k * nf : nullptr;
+        P->fl.adjB = bbuf ? bbuf + k * nf : nullptr;
+        P->fl.adjD = dbuf ? dbuf + k * D * nf : nullptr;
+        P->p_out = pbuf + k * nf;
+        P->fl.rhoi = P->fl.rhot;
+        if (nonlin) P->rhot_out = sbuf + k * nf;
+      }
+      r = enqueue_step(P, qend >= 0 && t >= qend, t - t0, t1 - t0);
+    }
+    restore_plan();
+    return r;
+  };
+  // forward pass: records the traces, keeps the state before every segment but the last,
+  // whose steps are reversed at once
   if ((rc = kw_plan_init(P))) return rc;
   P->t_host = -1;  // the sweep below sets the step counter itself
-  P->skip_gather = false;
-  for (int t = tb; t < nt; ++t) {
-    if ((t - tb) % ckpt == 0 && (rc = copy_state((t - tb) / ckpt, true))) return rc;
-    if ((rc = enqueue_step(P))) return rc;
+  for (int seg = 0; seg < nck; ++seg) {
+    if (seg < nck - 1 && (rc = copy_state(seg, true))) return rc;
+    if ((rc = run_segment(seg, seg == nck - 1))) return rc;
   }
   // reverse sweep, one checkpoint segment at a time
   for (float* f : {af.pb, af.cb, af.R}) KW_LAUNCH(launch_fill(f, nf, 0.f, P->st));
@@ -1189,48 +1230,33 @@ int kw_plan_adjoint_c(kw_plan* P, const float* adj, int ckpt, float* grad_c) {
     KW_LAUNCH(launch_fill(af.ub[i], nf, 0.f, P->st));
     KW_LAUNCH(launch_fill(af.rb[i], nf, 0.f, P->st));
   }
-  int* tdev = P->fl.tdev;
-  P->skip_gather = true;
   for (int seg = nck - 1; seg >= 0 && rc == KW_OK; --seg) {
     const int t0 = tb + seg * ckpt, t1 = std::min(nt, t0 + ckpt);
-    P->fl.tdev = tdev;
-    if ((rc = copy_state(seg, false))) break;
-    // a step starts from F_z[p], which the previous step's last kernel leaves in
-    // spectrum buffer 0: rebuild it from the restored p (same transform code)
-    if (launch_zfwd(g, nb, P->fl.p, g.ntot, P->fl.spec[0], g.nspec, P->ops.tw[D - 1], P->st) != hipSuccess) {
-      rc = fail(KW_EHIP, "adjoint: transform of the restored pressure failed");
-      break;
+    if (seg < nck - 1) {
+      if ((rc = copy_state(seg, false))) break;
+      // a step starts from F_z[p], which the previous step's last kernel leaves in
+      // spectrum buffer 0: rebuild it from the restored p (same transform code)
+      if (launch_zfwd(g, nb, P->fl.p, g.ntot, P->fl.spec[0], g.nspec, P->ops.tw[D - 1], P->st) != hipSuccess) {
+        rc = fail(KW_EHIP, "adjoint: transform of the restored pressure failed");
+        break;
+      }
+      if (launch_setint(tdev, nb, t0, P->st) != hipSuccess) { rc = fail(KW_EHIP, "adjoint: step counter reset failed"); break; }
+      P->skip_gather = true;
+      if ((rc = run_segment(seg, true))) break;
     }
-    if (launch_setint(tdev, nb, t0, P->st) != hipSuccess) { rc = fail(KW_EHIP, "adjoint: step counter reset failed"); break; }
-    if (nonlin && hipMemcpyAsync(sbuf, P->fl.rhot, sizeof(float) * nf, hipMemcpyDeviceToDevice, P->st) != hipSuccess) {
-      rc = fail(KW_EHIP, "adjoint: copy of the density sum failed");
-      break;
-    }
-    for (int t = t0; t < t1 && rc == KW_OK; ++t) {
-      P->fl.adjA = abuf ? abuf + (int64_t)(t - t0) * nf : nullptr;
-      P->fl.adjB = bbuf ? bbuf + (int64_t)(t - t0) * nf : nullptr;
-      P->fl.adjD = dbuf ? dbuf + (int64_t)(t - t0) * D * nf : nullptr;
-      if ((rc = enqueue_step(P))) break;
-      if (hipMemcpyAsync(pbuf + (int64_t)(t - t0) * nf, P->fl.p, sizeof(float) * nf, hipMemcpyDeviceToDevice, P->st) != hipSuccess)
-        rc = fail(KW_EHIP, "adjoint: copy of p failed");
-      else if (nonlin && hipMemcpyAsync(sbuf + (int64_t)(t - t0 + 1) * nf, P->fl.rhot, sizeof(float) * nf, hipMemcpyDeviceToDevice,
-                                        P->st) != hipSuccess)
-        rc = fail(KW_EHIP, "adjoint: copy of the density sum failed");
-    }
-    P->fl.adjA = P->fl.adjB = P->fl.adjD = nullptr;
     P->fl.tdev = nullptr;  // column passes of the reverse step must not skip instances at t = Nt
     for (int t = t1 - 1; t >= t0 && rc == KW_OK; --t) {
-      af.pt = pbuf + (int64_t)(t - t0) * nf;
-      af.At = abuf ? abuf + (int64_t)(t - t0) * nf : nullptr;
-      af.Bt = bbuf ? bbuf + (int64_t)(t - t0) * nf : nullptr;
-      af.St = sbuf ? sbuf + (int64_t)(t - t0 + 1) * nf : nullptr;
-      af.Sp = sbuf ? sbuf + (int64_t)(t - t0) * nf : nullptr;
-      af.Dt = dbuf ? dbuf + (int64_t)(t - t0) * D * nf : nullptr;
+      const int64_t k = t - t0;
+      af.pt = pbuf + k * nf;
+      af.At = abuf ? abuf + k * nf : nullptr;
+      af.Bt = bbuf ? bbuf + k * nf : nullptr;
+      af.St = sbuf ? sbuf + k * nf : nullptr;
+      af.Sp = !sbuf ? nullptr : k ? sbuf + (k - 1) * nf : rhot_state;
+      af.Dt = dbuf ? dbuf + k * D * nf : nullptr;
       rc = adjoint_step(P, af, Zbuf, t);
     }
+    P->fl.tdev = tdev;
   }
-  P->fl.tdev = tdev;
-  P->skip_gather = false;
   if (rc) { (void)hipStreamSynchronize(P->st); return rc; }
   if (with_p0) {  // the c-dependence of the set state: rho_i = p0 / (c0^2 p0div_i)
     for (int b = 0; b < nb && rc == KW_OK; ++b) {

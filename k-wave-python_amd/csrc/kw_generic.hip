@@ -666,7 +666,7 @@ __global__ __launch_bounds__(kGenThreads) void k_gcol(Geom g, Fields fl, Ops ops
              [&](int e) {
                const int n = e >> ls, col = min(col0 + (e & (L - 1)), a.ncols - 1);
                const float kx = k0[n], ky = k1[g.nd == 2 ? col : o], kz = w2 * k2[col];
-               const float f = sinc_poly(kap2 * fmaf(kx, kx, fmaf(kz, kz, ky * ky)));
+               const float f = sinc_k2<false>(kap2 * fmaf(kx, kx, fmaf(kz, kz, ky * ky)));
                return cscale(ld2(t, jb.axis == 0 ? n : ((jb.axis == 1 && g.nd == 3) ? o : col)), f);
              },
              put);
@@ -787,7 +787,7 @@ __device__ __forceinline__ GMassOps gmass_load(const Geom& g, const Fields& fl, 
   o.c2 = ld(I.c0sq, idx, I.c0sq_s);
   // (linear plans have neither array: the loads go to one that exists and are not used)
   const bool nl = flags & FLAG_NONLINEAR;
-  o.rs = gp(nl ? fl.rhot : fl.rho[0])[off + idx];
+  o.rs = gp(nl ? fl.rhoi : fl.rho[0])[off + idx];
   o.ba = ld(nl ? I.bona : I.rho0, idx, nl ? I.bona_s : I.rho0_s);
 #pragma unroll
   for (int i = 0; i < 3; ++i) {

@@ -596,7 +596,7 @@ __global__ __launch_bounds__(ZCfg<N>::NT) KW_WPE(N, KW_WPE_MASS) void k_mass(Geo
     rt[m] = make_float2(0.f, 0.f);
   }
   if (flags & FLAG_NONLINEAR) {
-    const auto rhot = gp(fl.rhot + off);
+    const auto rhot = gp(fl.rhoi + off);
     float2 ro[C::E];
 #pragma unroll
     for (int m = 0; m < C::E; ++m) ro[m] = make_float2(rhot[iA + m * C::TPL], rhot[iA + N + m * C::TPL]);
@@ -920,7 +920,13 @@ __global__ __launch_bounds__((ZCfg<N, NAR>::NT)) void k_src_build(Geom g, Fields
 // (no square root on the common path).  kappa = sinc(x) and cos(x) for
 // x = c_ref dt |k| / 2 from x^2: Taylor polynomials in x^2 up to x^2 = 4 (FP32
 // rounding), sin(x)/x and cos(x) beyond.
-__device__ __forceinline__ float sinc_poly(float x2) {
+// BIG = false: the caller has tested x^2 <= 4, for a whole line at once.
+template <bool BIG = true>
+__device__ __forceinline__ float sinc_k2(float x2) {
+  if (BIG && x2 > 4.f) {
+    const float x = sqrtf(x2);
+    return sinf(x) / x;
+  }
   float p = -1.f / 1307674368000.f;                 // -1/15!
   p = fmaf(p, x2, 1.f / 6227020800.f);              //  1/13!
   p = fmaf(p, x2, -1.f / 39916800.f);               // -1/11!
@@ -930,14 +936,9 @@ __device__ __forceinline__ float sinc_poly(float x2) {
   p = fmaf(p, x2, -1.f / 6.f);                      // -1/3!
   return fmaf(p, x2, 1.f);
 }
-__device__ __forceinline__ float sinc_k2(float x2) {
-  if (x2 > 4.f) {
-    const float x = sqrtf(x2);
-    return sinf(x) / x;
-  }
-  return sinc_poly(x2);
-}
-__device__ __forceinline__ float cos_poly(float x2) {
+template <bool BIG = true>
+__device__ __forceinline__ float cos_k2(float x2) {
+  if (BIG && x2 > 4.f) return cosf(sqrtf(x2));
   float p = -1.f / 87178291200.f;                   // -1/14!
   p = fmaf(p, x2, 1.f / 479001600.f);               //  1/12!
   p = fmaf(p, x2, -1.f / 3628800.f);                // -1/10!
@@ -947,7 +948,6 @@ __device__ __forceinline__ float cos_poly(float x2) {
   p = fmaf(p, x2, -0.5f);                           // -1/2!
   return fmaf(p, x2, 1.f);
 }
-__device__ __forceinline__ float cos_k2(float x2) { return x2 > 4.f ? cosf(sqrtf(x2)) : cos_poly(x2); }
 // |k|^a from |k|^2 for |k| > 0 (the fractional Laplacian is 0 at |k| = 0)
 __device__ __forceinline__ float kpow2(float km2, float a) { return km2 == 0.f ? 0.f : exp2f(0.5f * a * log2f(km2)); }
 
@@ -970,10 +970,10 @@ __device__ __forceinline__ void job_factor(int kind, float kap, const float (&km
       for (int m = 0; m < E; ++m) f[m] = kind == XK_SRCKAPPA ? cos_k2(k2 * km2[m]) : sinc_k2(k2 * km2[m]);
     } else if (kind == XK_SRCKAPPA) {
 #pragma unroll
-      for (int m = 0; m < E; ++m) f[m] = cos_poly(k2 * km2[m]);
+      for (int m = 0; m < E; ++m) f[m] = cos_k2<false>(k2 * km2[m]);
     } else {
 #pragma unroll
-      for (int m = 0; m < E; ++m) f[m] = sinc_poly(k2 * km2[m]);
+      for (int m = 0; m < E; ++m) f[m] = sinc_k2<false>(k2 * km2[m]);
     }
   } else {
 #pragma unroll
@@ -1475,7 +1475,7 @@ __global__ __launch_bounds__((ZCfg<N, true>::NT * ND)) void k_mass_small(Geom g,
   }
   if (flags & FLAG_NONLINEAR) {
 #pragma unroll
-    for (int m = 0; m < C::E; ++m) qv[m] = make_float2(gp(fl.rhot)[off + iA + m * C::TPL], gp(fl.rhot)[off + iA + N + m * C::TPL]);
+    for (int m = 0; m < C::E; ++m) qv[m] = make_float2(gp(fl.rhoi)[off + iA + m * C::TPL], gp(fl.rhoi)[off + iA + N + m * C::TPL]);
   }
   if (grp == ND - 1) {
 #pragma unroll

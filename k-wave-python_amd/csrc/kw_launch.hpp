@@ -40,6 +40,7 @@ hipError_t launch_gather(const Geom& g, int nb, int max_sens, const Fields& fl, 
 hipError_t launch_tick(const Fields& fl, const Inst* inst, int nb, int n, hipStream_t st);
 hipError_t launch_gather_tick(const Geom& g, int nb, int max_sens, const Fields& fl, const Inst* inst, int n, hipStream_t st);
 hipError_t launch_fill(float* p, int64_t n, float v, hipStream_t st);
+hipError_t launch_copies(const CopyList& c, int64_t n, hipStream_t st);
 hipError_t launch_setint(int* p, int n, int v, hipStream_t st);
 // surrogate (kw_fno.hip)
 hipError_t launch_mode_gemm(int M, int R, int N, int K, const uint16_t* A, const uint16_t* Bt, float* C, hipStream_t st);

@@ -34,6 +34,22 @@ __global__ void k_fill(float* __restrict__ p, int64_t n, float v) {
   if (i < n) p[i] = v;
 }
 
+// Copies of n floats, one per blockIdx.y (the state of the reverse sweep's checkpoints: a
+// copy command an array costs 4 us and its launch 10 at 64^3, eight arrays a checkpoint).
+__global__ void k_copies(CopyList c, int64_t n) {
+  const auto s = gp(c.src[blockIdx.y]);
+  const auto d = gw(c.dst[blockIdx.y]);
+  const int64_t step = (int64_t)gridDim.x * blockDim.x;
+  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += 4 * step) {
+    float v[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) v[k] = s[min(i + k * step, n - 1)];
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+      if (i + k * step < n) d[i + k * step] = v[k];
+  }
+}
+
 __global__ void k_setint(int* __restrict__ p, int n, int v) {
   for (int i = threadIdx.x; i < n; i += blockDim.x) p[i] = v;
 }
@@ -67,7 +83,9 @@ __global__ void k_adj_scatter(Geom g, AdjFields af, const Inst* __restrict__ ins
 // cbar += -(scale / c) sig(t) Z with Z = K R (additive) or R (uncorrected);
 // velocity along axis which: scale = 2 c dt / d_i (:636-642), so cbar += (scale / c)
 // sig(t) Z with Z = K U_i or U_i.  Zn is the unfiltered array (R or U_i), Zk the
-// filtered one.  One thread per grid row walks the row's source points (CSR).
+// filtered one.  Sixteen lanes take a grid row's source points (CSR; a row's points lie on
+// different columns): one thread a row spent 12.4 us of latencies on a 128^2 line source,
+// sixteen 3.0.
 __global__ void k_adj_srcgrad(Geom g, AdjFields af, int which, const float* __restrict__ Zn, const float* __restrict__ Zk,
                               const Inst* __restrict__ inst, int t) {
   const int b = blockIdx.y;
@@ -77,8 +95,10 @@ __global__ void k_adj_srcgrad(Geom g, AdjFields af, int which, const float* __re
   const float* Z = (s.mode == SRC_NOCORR ? Zn : Zk) + b * g.ntot;
   const float sgn = which < 0 ? -1.f : 1.f;
   float* cb = af.cb + b * g.ntot;
-  for (int r = blockIdx.x * blockDim.x + threadIdx.x; r < g.rows; r += gridDim.x * blockDim.x) {
-    for (int e = s.row_ptr[r]; e < s.row_ptr[r + 1]; ++e) {
+  const int lane = threadIdx.x % 16;
+  for (int64_t r = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) / 16; r < g.rows; r += (int64_t)gridDim.x * blockDim.x / 16) {
+    const int e1 = s.row_ptr[r + 1];
+    for (int e = s.row_ptr[r] + lane; e < e1; e += 16) {
       const int64_t idx = (int64_t)r * g.nz + s.col[e];
       const float c = sqrtf(I.c0sq[idx * I.c0sq_s]);
       const float sv = s.sig[(int64_t)s.sigrow[e] * s.len + t];
@@ -118,7 +138,7 @@ hipError_t launch_adj_scatter(const Geom& g, int nb, int max_sens, const AdjFiel
 
 hipError_t launch_adj_srcgrad(const Geom& g, int nb, const AdjFields& af, int which, const float* Zn, const float* Zk, const Inst* inst, int t,
                               hipStream_t st) {
-  hipLaunchKernelGGL(k_adj_srcgrad, dim3((g.rows + 255) / 256, nb), dim3(256), 0, st, g, af, which, Zn, Zk, inst, t);
+  hipLaunchKernelGGL(k_adj_srcgrad, dim3((unsigned)std::min<int64_t>((g.rows + 15) / 16, 65536), nb), dim3(256), 0, st, g, af, which, Zn, Zk, inst, t);
   return hipGetLastError();
 }
 
@@ -147,6 +167,13 @@ hipError_t launch_gather_tick(const Geom& g, int nb, int max_sens, const Fields&
 hipError_t launch_fill(float* p, int64_t n, float v, hipStream_t st) {
   if (n <= 0) return hipSuccess;
   hipLaunchKernelGGL(k_fill, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, p, n, v);
+  return hipGetLastError();
+}
+
+hipError_t launch_copies(const CopyList& c, int64_t n, hipStream_t st) {
+  if (n <= 0 || c.count <= 0) return hipSuccess;
+  const unsigned blocks = (unsigned)std::min<int64_t>((n + 1023) / 1024, 8192);
+  hipLaunchKernelGGL(k_copies, dim3(blocks, c.count), dim3(256), 0, st, c, n);
   return hipGetLastError();
 }
 

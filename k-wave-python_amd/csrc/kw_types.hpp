@@ -117,6 +117,7 @@ struct Fields {
   float* u[3];
   float* rho[3];
   float* rhot;
+  const float* rhoi;  // density sum of the previous step: rhot, or its slot of the reverse sweep's replay
   float2* spec[kMaxBufs];
   float* uc[3];     // velocity on the pressure grid (only when it is recorded)
   int* tdev;        // per-instance step counter
@@ -131,6 +132,12 @@ struct Fields {
   float* adjA;
   float* adjB;
   float* adjD;  // per-axis Dop_i u_i of the step, [nd][nb][ntot] (nonlinear adjoint replay)
+};
+
+struct CopyList {
+  const float* src[8];
+  float* dst[8];
+  int count;
 };
 
 // State of the reverse-time sweep of kw_plan_adjoint_c (all [nb][ntot] unless noted).
