@@ -85,7 +85,7 @@ def get_win(N, type_, plot_win=False, param=None, rotation=False, symmetric=True
         lin = np.squeeze(get_win(L, type_, param=param)[0])
         radius = (L - 1) / 2
         ll = np.linspace(-radius, radius, L)
-        grids = np.meshgrid(*[np.linspace(-radius, radius, int(n)) for n in Nb], indexing="ij")
+        grids = np.meshgrid(*[np.linspace(-radius, radius, int(n)) for n in Nb], indexing="ij", sparse=True)
         r = np.sqrt(sum(g ** 2 for g in grids))
         r[r > radius] = radius
         win = interp1d(ll, lin)(r)
