@@ -566,9 +566,10 @@ def predict(model, cmaps, batch=512, features=False, tta=False, ranges=False):
     device from the uploaded map.
 
     Host traffic: each batch of maps is copied into one of two page-locked staging
-    buffers and uploaded asynchronously, so that the copy of the next batch overlaps
-    the forward of the current one; the traces come back asynchronously into a
-    page-locked array that is returned as is (no further host copy)."""
+    buffers and uploaded on a stream of its own, so that both copies of the next batch
+    overlap the forward of the current one; the traces come back on a third stream, under
+    the next forward, into a page-locked array that is returned as is (no further host
+    copy).  1024 maps, one stream -> three: 6.4 -> 4.8 ms."""
     import torch
 
     dev = next(model.parameters()).device
@@ -576,39 +577,80 @@ def predict(model, cmaps, batch=512, features=False, tta=False, ranges=False):
     n = len(cm)
     src = torch.from_numpy(cm)
     stream = torch.cuda.current_stream(dev)
-    stage = [torch.empty((min(batch, n),) + cm.shape[1:], dtype=torch.float32, pin_memory=True) for _ in range(2)]
-    uploaded = [None, None]
+    up, down = torch.cuda.Stream(dev), torch.cuda.Stream(dev)
+    shape = (min(batch, n),) + cm.shape[1:]
+    starts = list(range(0, n, batch))
+    stage = [torch.empty(shape, dtype=torch.float32, pin_memory=True) for _ in starts[:2]]
+    maps = [torch.empty(shape, dtype=torch.float32, device=dev) for _ in starts[:2]]
+    up.wait_stream(stream)  # (what used these blocks before)
+    uploaded, used = [None, None], [None, None]
     out, fts, rng = None, [], []
-    with torch.no_grad(), torch.autocast("cuda", dtype=torch.bfloat16):
-        for k, i in enumerate(range(0, n, batch)):
-            nb = min(batch, n - i)
-            buf = stage[k % 2]
-            if uploaded[k % 2] is not None:
-                uploaded[k % 2].synchronize()  # the upload from this buffer two batches ago has finished
-            buf[:nb].copy_(src[i:i + nb])
-            x = buf[:nb].to(dev, non_blocking=True)
-            uploaded[k % 2] = torch.cuda.Event()
-            uploaded[k % 2].record(stream)
-            if ranges:
-                flat = x.reshape(nb, -1)
-                rng.append(torch.stack([flat.amin(1), flat.amax(1)], 1))
-            r = model(torch.cat([x, x.flip(-1)]) if tta else x, features=features)
-            if features:
-                r, f = r
-                f = f.float()
-            r = r.float()
-            if tta:
-                a, m = r[:nb], r[nb:].flip(1)
-                r = 0.5 * (a + m)
+
+    def upload(k):
+        """Batch k into its staging buffer and on to the device, in pieces: the first starts early."""
+        i, j = starts[k], k % 2
+        nb = min(batch, n - i)
+        if uploaded[j] is not None:
+            uploaded[j].synchronize()  # the upload from this buffer two batches ago has finished
+        with torch.cuda.stream(up):
+            if used[j] is not None:
+                up.wait_event(used[j])  # the forward two batches ago has read its maps
+            for a in range(0, nb, 128):
+                b = min(a + 128, nb)
+                stage[j][a:b].copy_(src[i + a:i + b])
+                maps[j][a:b].copy_(stage[j][a:b], non_blocking=True)
+            uploaded[j] = up.record_event()
+
+    def download(r, i, ready):
+        down.wait_event(ready)
+        with torch.cuda.stream(down):
+            out[i:i + len(r)].copy_(r, non_blocking=True)
+        r.record_stream(down)
+
+    # Order of enqueueing: a copy that is enqueued behind a download that still waits for its
+    # forward does not start before that download has ended, so a batch's upload goes ahead of
+    # the forward before it, and a batch's download behind the forward after it.
+    done = None
+    try:
+        if n:
+            upload(0)
+        with torch.no_grad(), torch.autocast("cuda", dtype=torch.bfloat16):
+            for k, i in enumerate(starts):
+                nb = min(batch, n - i)
+                ready = uploaded[k % 2]
+                if k + 1 < len(starts):
+                    upload(k + 1)
+                stream.wait_event(ready)
+                x = maps[k % 2][:nb]
+                if ranges:
+                    flat = x.reshape(nb, -1)
+                    rng.append(torch.stack([flat.amin(1), flat.amax(1)], 1))
+                r = model(torch.cat([x, x.flip(-1)]) if tta else x, features=features)
                 if features:
-                    dis = (a - m).flatten(1).norm(dim=1) / r.flatten(1).norm(dim=1).clamp_min(1e-30)
-                    f = torch.cat([f[:nb], torch.log10(dis.clamp_min(1e-12))[:, None]], 1)
-            r = r * TRACE_SCALE
-            if out is None:
-                out = torch.empty((n,) + tuple(r.shape[1:]), dtype=torch.float32, pin_memory=True)
-            out[i:i + nb].copy_(r, non_blocking=True)
-            if features:
-                fts.append(f)
+                    r, f = r
+                    f = f.float()
+                r = r.float()
+                if tta:
+                    a, m = r[:nb], r[nb:].flip(1)
+                    r = 0.5 * (a + m)
+                    if features:
+                        dis = (a - m).flatten(1).norm(dim=1) / r.flatten(1).norm(dim=1).clamp_min(1e-30)
+                        f = torch.cat([f[:nb], torch.log10(dis.clamp_min(1e-12))[:, None]], 1)
+                r = r * TRACE_SCALE
+                used[k % 2] = stream.record_event()
+                if out is None:
+                    out = torch.empty((n,) + tuple(r.shape[1:]), dtype=torch.float32, pin_memory=True)
+                if done is not None:
+                    download(*done)
+                done = (r, i, used[k % 2])
+                if features:
+                    fts.append(f)
+            if done is not None:
+                download(*done)
+    finally:
+        # the maps' and the traces' memory goes back to the caller's stream
+        stream.wait_stream(up)
+        stream.wait_stream(down)
     stream.synchronize()
     res = [out.numpy()]
     if features:

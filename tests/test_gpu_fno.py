@@ -319,3 +319,72 @@ def test_head_gather_matches_index_select():
     got = head_gather(v, cols.cuda())
     want = v.permute(0, 3, 1, 2).index_select(1, cols.long().cuda())
     assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("p", [4, 60, 132, 4096, 4100])  # tiles of 64 positions a wavefront, 256 a workgroup
+def test_pointwise_on_the_matrix_cores_covers_ragged_tiles(p):
+    """32 channels run on FP32 matrix instructions: no weight or sum is rounded below FP32, so
+    one bf16 rounding (2^-9 of the value, to nearest) is all that separates the result from
+    FP64; a sum that lies on a rounding boundary may fall to either side, hence 2^-8."""
+    import torch
+
+    from kwave_amd.surrogate import fno_pointwise
+
+    g = torch.Generator().manual_seed(p)
+    v = torch.randn(3, 32, p, generator=g).to("cuda", torch.bfloat16)
+    s = torch.randn(3, 32, p, generator=g).to("cuda", torch.bfloat16)
+    pw = (torch.randn(32, 32, generator=g) / 32 ** 0.5).cuda()
+    pb = torch.randn(32, 1, generator=g).cuda()
+    out = fno_pointwise(v, s, pw, pb, False).double()
+    ref = s.double() + pb.double() + torch.matmul(pw.double(), v.double())
+    assert float(((out - ref).abs() - 2.0 ** -8 * ref.abs()).max()) <= 1e-6
+
+
+@pytest.mark.parametrize("slabs", [1, 2, 3, 5000])  # more than two rounds of any resident grid: every prefetch
+def test_dft_kernels_do_not_depend_on_the_number_of_slabs(slabs):
+    import torch
+
+    from kwave_amd.surrogate import fno_dft
+
+    mxb, mytb, nytb, nxb = _dft_operands()[4:]
+    g = torch.Generator().manual_seed(slabs)
+    few = torch.randn(5, 64, 64, generator=g).to("cuda", torch.bfloat16)
+    modes = torch.randn(5, 32, 32, generator=g).cuda()
+    pick = torch.arange(slabs) % 5
+    for d, x, m in ((1, few, (mxb, mytb)), (-1, modes, (nytb, nxb))):
+        one = torch.stack([fno_dft(d, x[i:i + 1].contiguous(), *m)[0] for i in range(5)])
+        assert torch.equal(fno_dft(d, x[pick].contiguous(), *m), one[pick])
+
+
+def test_head_gather_of_misaligned_slabs():
+    """2-byte accesses where the slabs are not 16-byte aligned."""
+    import torch
+
+    from kwave_amd.surrogate import head_gather
+
+    flat = torch.randn(1 + 2 * 3 * 64 * 64, generator=torch.Generator().manual_seed(6)).to("cuda", torch.bfloat16)
+    v = flat[1:].view(2, 3, 64, 64)
+    cols = torch.tensor([7, 0, 63], dtype=torch.int32)
+    want = v.permute(0, 3, 1, 2).index_select(1, cols.long().cuda())
+    assert v.data_ptr() % 16 and torch.equal(head_gather(v, cols.cuda()), want)
+
+
+@pytest.mark.parametrize("n,batch", [(1, 512), (6, 3), (11, 3)])  # the staging buffers are used up to twice each
+@pytest.mark.parametrize("tta", [False, True])
+def test_predict_pipeline_gives_the_forward_of_each_batch(n, batch, tta):
+    import torch
+
+    from kwave_amd import surrogate as S
+
+    torch.manual_seed(2)
+    model = S.build_model()
+    maps = (1400 + 250 * torch.rand(n, 128, 128, generator=torch.Generator().manual_seed(n))).numpy()
+    got, rng = S.predict(model, maps, batch=batch, tta=tta, ranges=True)
+    want = []
+    with torch.no_grad(), torch.autocast("cuda", dtype=torch.bfloat16):
+        for i in range(0, n, batch):
+            x = torch.from_numpy(maps[i:i + batch]).cuda()
+            r = model(torch.cat([x, x.flip(-1)]) if tta else x).float()
+            want.append((0.5 * (r[: len(x)] + r[len(x):].flip(1)) if tta else r) * S.TRACE_SCALE)
+    assert np.array_equal(got, torch.cat(want).cpu().numpy())
+    assert np.array_equal(rng, np.stack([maps.min((1, 2)), maps.max((1, 2))], 1))
