@@ -1401,11 +1401,15 @@ int batch_graph(kw_batch* B, int k, const std::string& form, hipGraphExec_t* out
   KW_HIP(hipStreamBeginCapture(B->st, hipStreamCaptureModeThreadLocal));
   int rc = KW_OK;
   hipError_t e = hipEventRecord(B->fork, B->st);
+  const bool shared = std::count(form.begin(), form.end(), '-') + 1 < (int64_t)form.size();  // more than one plan runs
   for (size_t i = 0; i < B->plans.size() && rc == KW_OK && e == hipSuccess; ++i) {
     if (form[i] == '-') continue;
     kw_plan* P = B->plans[i];
     e = hipStreamWaitEvent(P->st, B->fork, 0);
+    const int small = P->g.small;
+    if (shared && small == 1) P->g.small = 3;
     for (int s = 0; s < k && rc == KW_OK && e == hipSuccess; ++s) rc = enqueue_step(P, form[i] == 'l', s, k);
+    P->g.small = small;
     if (rc == KW_OK && e == hipSuccess) e = hipEventRecord(B->join[i], P->st);
     if (rc == KW_OK && e == hipSuccess) e = hipStreamWaitEvent(B->st, B->join[i], 0);
   }

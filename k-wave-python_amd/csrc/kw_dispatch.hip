@@ -12,10 +12,11 @@ namespace kw {
 // step with the large-grid forms -> with the small ones: 256^2 35.6 -> 30.1, 64 maps of
 // 128^2 (66 k lanes a group) 64.1 -> 59.9, 1024^2 power law 109.8 -> 103.1; beyond, the sixteen
 // scan lines of 256^2 to 640^2 lose (197.7 -> 201.6 at 150 k lanes, 218.5 at 300 k) and
-// 160^3 (512 k lanes an axis) 289 -> 324.
+// 160^3 (512 k lanes an axis) 289 -> 324.  Plans of a batch share the chip with the others'
+// kernels and take half as many (small 3): the scan lines 176 -> 163 us a step.
 bool z_small(const Geom& g, int nb, int tpl, int groups) {
   if (g.small == 0) return false;
-  return g.small == 2 || (int64_t)(g.rows / 2) * tpl * nb * groups <= 150000;
+  return g.small == 2 || (int64_t)(g.rows / 2) * tpl * nb * groups <= (g.small == 3 ? 75000 : 150000);
 }
 
 #define KW_DECL4(RET, NAME, ...) \

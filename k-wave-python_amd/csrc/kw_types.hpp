@@ -22,7 +22,7 @@ struct Geom {
   int rows;          // ntot / nz
   int64_t ntot;      // real elements per instance
   int64_t nspec;     // rows * nhp complex elements per instance (storage)
-  int small;         // small-grid forms of the contiguous-axis kernels: 0 never, 1 by the size rule (z_small), 2 always
+  int small;         // small-grid forms of the contiguous-axis kernels: 0 never, 1 by the size rule (z_small), 2 always, 3 by the rule of a batch of plans
 };
 
 // One time-varying source term (p, or one velocity component).
