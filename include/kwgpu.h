@@ -201,8 +201,8 @@ int kw_plan_destroy(kw_plan* plan);
  * lossless or with Stokes or power-law absorption (with or without dispersion),
  * with or without B/A nonlinearity (kspace_solver.py:542-550); every
  * instance records p with a common Nt, sensor count and record start.  The plan's fields
- * and records afterwards are those of the forward run's first segment replay:
- * call kw_plan_init before stepping it again.  The reference has no adjoint:
+ * afterwards are those at the end of the forward run's first segment, its records those
+ * of the whole run: call kw_plan_init before stepping it again.  The reference has no adjoint:
  * this differentiates its Simulation.step (kspace_solver.py:691-747) and source
  * scaling (:619-624). */
 int kw_plan_adjoint_c(kw_plan* plan, const float* adj, int ckpt, float* grad_c);

@@ -1257,6 +1257,18 @@ int kw_plan_adjoint_c(kw_plan* P, const float* adj, int ckpt, float* grad_c) {
     }
     P->fl.tdev = tdev;
   }
+  if (rc == KW_OK && nck > 0) {
+    // the first segment's replay left its last p and density sum in their slots: back to the
+    // plan's buffers, beside the u_i and rho_i of the same step
+    const int64_t k = std::min(ckpt, nt - tb) - 1;
+    CopyList c{};
+    c.count = nonlin ? 2 : 1;
+    c.src[0] = pbuf + k * nf;
+    c.dst[0] = p_state;
+    c.src[1] = nonlin ? sbuf + k * nf : nullptr;
+    c.dst[1] = rhot_state;
+    if (launch_copies(c, nf, P->st) != hipSuccess) rc = fail(KW_EHIP, "adjoint: copy of the replayed fields failed");
+  }
   if (rc) { (void)hipStreamSynchronize(P->st); return rc; }
   if (with_p0) {  // the c-dependence of the set state: rho_i = p0 / (c0^2 p0div_i)
     for (int b = 0; b < nb && rc == KW_OK; ++b) {

@@ -274,3 +274,26 @@ def test_torch_autograd_matches_adjoint():
     loss.backward()
     g_ref, _ = _gpu_grad(case, (y.detach() - d).numpy(), checkpoint=30)
     assert np.array_equal(c.grad.numpy(), g_ref)
+
+
+@pytest.mark.parametrize("shape,nt,p0,kw", [((32, 40), 50, True, {}), ((16, 24, 32), 40, False, NONLINEAR),
+                                            ((30, 22), 40, True, dict(NONLINEAR, alpha=ABSORBING["powerlaw-mild"]))])
+@pytest.mark.parametrize("checkpoint", [7, 200])  # several segments and one
+def test_fields_after_the_adjoint_are_the_first_segments(shape, nt, p0, kw, checkpoint):
+    """p, u_i and rho_i belong to one step: the last of the first segment, as kwgpu.h says."""
+    from kwave_amd import _abi
+    from kwave_amd.solvers.plan import DevicePlan
+    from kwave_amd.solvers.setup import build_instance
+
+    kg, med, src, sen, pml, alpha = adjoint_case(shape=shape, nt=nt, p0=p0, **kw)
+    pl = DevicePlan([build_instance(kg, med, copy.deepcopy(src), sen, pml_size=pml, pml_alpha=alpha)])
+    fields = [_abi.F_P] + [f + i for f in (_abi.F_UX, _abi.F_RHOX) for i in range(len(shape))]
+    pl.adjoint_c([np.ones((int(sen.mask.sum()), nt), dtype=np.float32)], checkpoint=checkpoint)
+    step, got = pl.step_index(0), [pl.field(0, f) for f in fields]
+    assert step == min(nt, checkpoint + int(p0))
+    pl.reset()
+    pl.run(step - pl.step_index(0))
+    for f, a in zip(fields, got):
+        want = pl.field(0, f)
+        assert np.abs(want).max() > 0 and np.array_equal(a, want), f
+    pl.close()
