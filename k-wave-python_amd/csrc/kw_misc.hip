@@ -17,14 +17,14 @@ __global__ void k_tick(Fields fl, const Inst* __restrict__ inst, int nb, int n) 
   for (int b = threadIdx.x; b < nb; b += blockDim.x) fl.tdev[b] = min(fl.tdev[b] + n, max(fl.tdev[b], inst[b].nt));
 }
 
-// both, for instances with few sensors: one workgroup an instance, which reads the
-// counter before it advances it
-__global__ __launch_bounds__(256) void k_gather_tick(Geom g, Fields fl, const Inst* __restrict__ inst, int n) {
+// both, for instances with few sensors: one workgroup an instance, a lane a sensor, which
+// reads the counter before it advances it
+constexpr int kGatherTickSensors = 256;
+__global__ __launch_bounds__(kGatherTickSensors) void k_gather_tick(Geom g, Fields fl, const Inst* __restrict__ inst, int n) {
   const int b = blockIdx.x;
   const Inst& I = inst[b];
-  const int t0 = fl.tdev[b], t = t0 + fl.toff;
-  if (t < I.nt)
-    for (int s = threadIdx.x; s < I.nsens; s += blockDim.x) gather_point(g, fl, I, b, t, s);
+  const int t0 = fl.tdev[b];
+  gather_point(g, fl, I, b, t0 + fl.toff, threadIdx.x);
   __syncthreads();
   if (threadIdx.x == 0) fl.tdev[b] = min(t0 + n, max(t0, I.nt));
 }
@@ -154,13 +154,18 @@ hipError_t launch_tick(const Fields& fl, const Inst* inst, int nb, int n, hipStr
   return hipGetLastError();
 }
 
-// one launch for both up to 4096 sensors (16 a thread)
+// One launch for both while every point has a lane of the one workgroup: beyond, its points
+// follow each other, each a chain of latencies, where k_gather spreads them over the chip.  us a
+// single step, one launch -> two: 128^2 p at 256 points 28.8 -> 30.1, at 512 29.7 -> 30.1, at 1000
+// 31.3 -> 30.1, at 3000 37.1 -> 30.2; p and u at 256 37.7 -> 39.0, at 512 39.6 -> 39.2; 96^3 p
+// and u at 256 167.2 -> 168.7, at 512 170.2 -> 168.8, at 1000 175.8 -> 168.7; p interpolated over
+// eight corners at 256 115.5 -> 116.4, at 500 119.4 -> 117.4, at 1500 132.2 -> 117.2.
 hipError_t launch_gather_tick(const Geom& g, int nb, int max_sens, const Fields& fl, const Inst* inst, int n, hipStream_t st) {
-  if (max_sens > 4096) {
+  if (max_sens > kGatherTickSensors) {
     const hipError_t e = launch_gather(g, nb, max_sens, fl, inst, st);
     return e != hipSuccess ? e : launch_tick(fl, inst, nb, n, st);
   }
-  hipLaunchKernelGGL(k_gather_tick, dim3(nb), dim3(256), 0, st, g, fl, inst, n);
+  hipLaunchKernelGGL(k_gather_tick, dim3(nb), dim3(kGatherTickSensors), 0, st, g, fl, inst, n);
   return hipGetLastError();
 }
 
