@@ -327,8 +327,8 @@ __device__ __forceinline__ void set_lane(float2 (&a)[E], int m, int h, float v) 
 // nonlinear flag, a source mode, a clamped row) had compiled into one block per element,
 // each load waited for alone.  Straight-line loops with the tests around them took the
 // mass kernel from 1970 to 1686 us at 512^3 and from 264 to 187 us at 256^3, eos from 902
-// to 811 and from 126 to 102 us, momentum from 198 to 186 us at 256^3 (1751 -> 1846 at
-// 512^3), and 256^3 steps from 1287 to 1159 us.
+// to 811 and from 126 to 102 us, momentum from 198 to 186 us at 256^3, and 256^3 steps from
+// 1287 to 1159 us.  Momentum has a second order of its loads for larger grids (kMomStaged).
 #ifndef KW_WPE_MOM
 #define KW_WPE_MOM 1
 #endif
@@ -490,12 +490,20 @@ __device__ __forceinline__ void pml_rows(const float* const* tab, const Geom& g,
 // momentum: u_i = pml_sg (pml_sg u_i - dt/rho0_sg * grad_i p) (+ source), then
 // forward transform of u_i along z (for the divergence).  blockIdx.z = axis.
 // ---------------------------------------------------------------------------
-template <int N>
+// STAGED (rule kMomStaged): the tables are in LDS before the operands are loaded.
+template <int N, bool STAGED>
 __global__ __launch_bounds__(ZCfg<N>::NT) KW_WPE(N, KW_WPE_MOM) void k_momentum(Geom g, Fields fl, const Inst* __restrict__ inst, const float2* __restrict__ tw_g) {
   const int ax = blockIdx.z;
   const bool zax = ax == g.nd - 1;
-  KW_ZPASS_EARLY(zax ? inst[blockIdx.y].pmlsg[ax] : nullptr)
+  KW_ZPASS_EARLY(!STAGED && zax ? inst[blockIdx.y].pmlsg[ax] : nullptr)
   const int t = step_of(fl, b);
+  if constexpr (STAGED) {
+    if (t >= I.nt) return;
+    put_stage_tw<N, C::PV, C::NT>(twr, twl, tid);
+    __syncthreads();
+    if (zax)
+      for (int i = tid; i < N; i += C::NT) pmlz[i] = gp(I.pmlsg[ax])[i];
+  }
   KW_ROWS_CLAMPED
   float2* sp = fl.spec[ax] + b * g.nspec;
   const auto u = gw(fl.u[ax] + b * g.ntot);
@@ -512,8 +520,12 @@ __global__ __launch_bounds__(ZCfg<N>::NT) KW_WPE(N, KW_WPE_MOM) void k_momentum(
   }
   float2 gv[C::E], As[C::IT], Bs[C::IT];
   pair_load<C>(As, Bs, sp, row0, rows, g.nhp, tid);
-  if (t >= I.nt) return;
-  KW_ZPASS_PUT
+  if constexpr (STAGED) {
+    __syncthreads();
+  } else {
+    if (t >= I.nt) return;
+    KW_ZPASS_PUT
+  }
   pair_put<C>(lds, As, Bs, tid);
   inv_from_lds<C>(lds, tw, tid, gv);
   const int smode = src_mode_at(src, t);
