@@ -10,25 +10,21 @@ namespace kw {
 
 constexpr int kColDevices = 64;
 
-// Workgroups of k_col<S, L, OPS> resident on the current device at once (0 if
-// the runtime cannot say).  Queried once per kernel and device.
+// Workgroups of k_col<S, L, OPS> resident on the current device at once, at most
+// `most` per compute unit (0 if the runtime cannot say).  Queried once per kernel and device.
 template <int S, int L, bool OPS, int PV>
-static int col_resident() {
+static int col_resident(int most) {
   static std::mutex mu;
-  static int per_dev[kColDevices] = {};
+  static struct { int per_cu, cus; } per_dev[kColDevices] = {};
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kColDevices) return 0;
   std::lock_guard<std::mutex> lock(mu);
-  if (per_dev[dev] == 0) {
-    int per_cu = 0, cus = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, reinterpret_cast<const void*>(&k_col<S, L, OPS, 1, PV>),
-                                                     ColCfg<S, L, 1, PV>::NT, 0) != hipSuccess ||
-        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
-      per_dev[dev] = -1;
-    else
-      per_dev[dev] = per_cu > 0 && cus > 0 ? per_cu * cus : -1;
-  }
-  return per_dev[dev] > 0 ? per_dev[dev] : 0;
+  auto& d = per_dev[dev];
+  if (d.per_cu == 0 && (hipOccupancyMaxActiveBlocksPerMultiprocessor(&d.per_cu, reinterpret_cast<const void*>(&k_col<S, L, OPS, 1, PV>),
+                                                                     ColCfg<S, L, 1, PV>::NT, 0) != hipSuccess ||
+                        hipDeviceGetAttribute(&d.cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || d.per_cu <= 0))
+    d.per_cu = -1;
+  return d.per_cu > 0 ? std::min(d.per_cu, most) * d.cus : 0;
 }
 
 // Workgroups per instance of a column pass: every tile its own workgroup, or -
@@ -38,11 +34,19 @@ static int col_resident() {
 // loop (bit 0 those with spectral jobs, bit 1 the FFT-only ones); a.grid > 0
 // sets the looping grid (tests).  Results do not depend on either: every column
 // is transformed the same way.
+//
+// FFT-only passes over lengths with a factor 3 (E = 12) loop on three waves a SIMD, not the four
+// their registers allow, once a buffer exceeds 27 MB (the L2s hold 32).  us a y-pass, four ->
+// three: 384^3 280 -> 258, 192^3 39.0 -> 36.7, 256 x 384 x 128 68 -> 64, 512 x 48 x 512 55 -> 48,
+// 256 x 192 x 160 42.5 -> 36.8, 512 x 96 x 256 56.5 -> 58.4; below, 64 x 192 x 512 (25 MB)
+// 27.9 -> 33.3, 96 x 96 x 512 21.0 -> 23.5.  With a factor 5 three lose (320^3 149 -> 173).
 template <int S, int L, bool OPS, int PV>
 static int col_grid(const ColArgs& a, int tiles, int nb) {
+  using C = ColCfg<S, L, 1, PV>;
   if (!(a.persist & (OPS ? 1 : 2))) return tiles;
   if (a.grid > 0) return std::min(tiles, a.grid);
-  const int res = col_resident<S, L, OPS, PV>();
+  const bool three = !OPS && C::E == 12 && (int64_t)sizeof(float2) * a.nouter * a.ncols * S * nb > 27000000;
+  const int res = col_resident<S, L, OPS, PV>(three ? std::max(1, 12 * 64 / C::NT) : 1 << 20);
   if (res <= 0 || (int64_t)tiles * nb <= res) return tiles;
   const int per = std::max(8, (res / nb) & ~7);
   return std::min(tiles, per);
