@@ -160,3 +160,34 @@ def test_plan_refuses_mixed_alpha_power():
         sts.append(build_instance(kg, med, src, sen, pml_size=pml, pml_alpha=alpha))
     with pytest.raises(ValueError, match="alpha_power"):
         DevicePlan(sts)
+
+
+def test_smoothing_threads_follow_the_process_affinity(monkeypatch):
+    """A pinned process (one of several ranks, a job on a share of the machine) starts no more
+    threads than it has processors; the result does not depend on their number."""
+    import os
+
+    import scipy.fft
+
+    from kwave_amd.utils import filters
+
+    counts = []
+
+    def spy(f):
+        def call(*args, workers=None, **kw):
+            counts.append(workers)
+            return f(*args, workers=workers, **kw)
+        return call
+
+    monkeypatch.setattr(filters.scipy.fft, "rfftn", spy(scipy.fft.rfftn))
+    monkeypatch.setattr(filters.scipy.fft, "irfftn", spy(scipy.fft.irfftn))
+    a = np.random.default_rng(0).random((24, 31, 18))
+    mine = os.sched_getaffinity(0)
+    wide = filters.smooth(a)
+    try:
+        os.sched_setaffinity(0, {min(mine)})
+        narrow = filters.smooth(a)
+    finally:
+        os.sched_setaffinity(0, mine)
+    assert counts == [min(8, len(mine))] * 2 + [1, 1]
+    assert np.array_equal(wide, narrow)
