@@ -33,7 +33,8 @@ def smooth(a, restore_max=False, window_type="Blackman"):
         # enough (with the window: 64^3 12.1 -> 4.1 ms, 256^3 858 -> 245 ms)
         if sq.dtype.itemsize < 8 or sq.dtype.kind != "f":
             sq = sq.astype(np.float64)
-        workers = min(8, len(os.sched_getaffinity(0)))
+        affinity = getattr(os, "sched_getaffinity", None)  # (Linux)
+        workers = min(8, len(affinity(0)) if affinity else os.cpu_count() or 1)
         half = scipy.fft.rfftn(sq, workers=workers)
         half *= shifted[..., : half.shape[-1]]
         out = scipy.fft.irfftn(half, s=shape, workers=workers, overwrite_x=True).reshape(orig)
