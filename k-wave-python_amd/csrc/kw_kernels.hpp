@@ -1380,6 +1380,7 @@ __global__ __launch_bounds__((ColCfg<N, L>::NT * (OPS ? kColSmallJobs : 1))) voi
 #define KW_ZSMALL_PROLOGUE(GROUPS)                                                                    \
   using C = ZCfg<N, true>;                                                                            \
   constexpr int G = GROUPS;                                                                           \
+  static_assert(C::NT % 64 == 0, "a group is whole wavefronts");                                      \
   __shared__ float2 lds_all[G][C::LDS];                                                               \
   __shared__ float2 twl[stage_tw_size<N, C::PV>()];                                                   \
   const int grp = __builtin_amdgcn_readfirstlane((int)threadIdx.x / C::NT);                           \

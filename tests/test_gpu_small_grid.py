@@ -148,3 +148,29 @@ def test_the_momentum_order_of_large_grids_gives_the_same_bits(shape, monkeypatc
 
     for a, b in zip(run("1"), run("2")):  # "2": the small-grid form at any size
         assert np.abs(a).max() > 0 and np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("shape", [(24, 16, 56), (16, 24, 112), (16, 16, 224), (24, 16, 448), (16, 16, 1024)])
+@pytest.mark.parametrize("absorb,bona", [(None, None), ((0.02, 2.0), 6.0), ((0.5, 1.3), 6.0)])
+def test_small_grid_forms_of_the_longest_rows_in_3d(shape, absorb, bona, monkeypatch):
+    """Three groups of lanes where their exchanges take the most LDS (fourteen elements a lane)
+    and, at 1024, two wavefronts a group: the step's forms and the reverse sweep's."""
+    from kwave_amd.adjoint import sound_speed_gradient
+    from kwave_amd.solvers.kspace_solver import Simulation
+
+    kg, med, src, sen = _case(shape, absorb, bona)
+    pml = dict(pml_size=(3,) * 3, pml_alpha=(2.0,) * 3)
+    adj = np.random.default_rng(3).standard_normal((int(sen.mask.sum()), 24)).astype(np.float32)
+
+    def run(form):
+        monkeypatch.setenv("KW_COL_SMALL", form)
+        monkeypatch.setenv("KW_Z_SMALL", form)
+        out = Simulation(kg, med, copy.deepcopy(src), sen, **pml).run()
+        sen_p = copy.deepcopy(sen)
+        sen_p.record = ["p"]
+        out["gradient"] = sound_speed_gradient(kg, med, copy.deepcopy(src), sen_p, adj, checkpoint=7, **pml)[0]
+        return out
+
+    large = run("0")
+    for k, v in run("2").items():
+        assert np.abs(large[k]).max() > 0 and np.array_equal(v, large[k]), k
