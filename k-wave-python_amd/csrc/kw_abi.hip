@@ -276,6 +276,13 @@ double zbytes_eos(const kw_plan* P) {
   return b;
 }
 
+// Sensors of all instances beyond which every step gathers its own in a kernel: inside a column
+// pass they run on that pass's registers and LDS, a few workgroups a compute unit.  us a step,
+// in the pass -> own kernel: 128^3 every cell (2.1 M) 141.1 -> 143.3, 1024^2 every cell 64.1 ->
+// 68.6; 128 x 256 x 256 half of the cells (4.2 M) 440.3 -> 436.4 and all 468 -> 455, 200 x 180 x
+// 170 all (6.1 M) 699.8 -> 676.9, 256^3 half (8 M) 852.7 -> 831.9.
+constexpr int64_t kGatherInPass = 3000000;
+
 // One time step.  lean: every spectral (CHAIN) and pattern pressure source
 // has ended, so no source spectrum is built or carried through the column
 // passes and the mass update takes its form without a staged source term.
@@ -283,14 +290,16 @@ double zbytes_eos(const kw_plan* P) {
 // Step j of a block of k: the device step counters stand at the block's first step and
 // are advanced once, by k, at its end.  Every step after the block's first gathers the
 // sensors of the step before it in its first column pass (ColArgs::gath); the last
-// gathers its own before the counters advance, so a block leaves nothing behind.
+// gathers its own before the counters advance, so a block leaves nothing behind (with very
+// many sensors every step gathers its own: kGatherInPass).
 int enqueue_step(kw_plan* P, bool lean = false, int j = 0, int k = 1) {
   const Geom& g = P->g;
   const int D = g.nd;
   const float2* twz = P->ops.tw[D - 1];
   int rc;
   P->fl.toff = j;
-  const int gath = j > 0 && !P->skip_gather ? P->max_sens : 0;
+  const bool own_gather = (int64_t)P->nb * P->max_sens > kGatherInPass && !P->skip_gather;
+  const int gath = j > 0 && !P->skip_gather && !own_gather ? P->max_sens : 0;
   // --- momentum: grad p, u update, F_z[u_i] ---
   std::vector<int> ub;
   std::vector<XJob> jobs;
@@ -344,8 +353,9 @@ int enqueue_step(kw_plan* P, bool lean = false, int j = 0, int k = 1) {
     if ((rc = ypass(P, 1, yb))) return rc;
     KW_TLAUNCH(KK_EOS, zbytes_eos(P), launch_eos(g, P->nb, P->fl, P->d_inst, twz, P->flags, P->st));
   }
+  if (own_gather) KW_TLAUNCH(KK_GATHER, 0.0, launch_gather(g, P->nb, P->max_sens, P->fl, P->d_inst, P->st));
   if (j == k - 1) {
-    if (P->skip_gather) KW_TLAUNCH(KK_TICK, 0.0, launch_tick(P->fl, P->d_inst, P->nb, k, P->st));
+    if (P->skip_gather || own_gather) KW_TLAUNCH(KK_TICK, 0.0, launch_tick(P->fl, P->d_inst, P->nb, k, P->st));
     else KW_TLAUNCH(KK_GATHER, 0.0, launch_gather_tick(g, P->nb, P->max_sens, P->fl, P->d_inst, k, P->st));
   }
   P->fl.toff = 0;

@@ -2,7 +2,8 @@
 
 A block of steps gathers in the column passes of the steps after the first and, for the
 last one, in a kernel that also advances the step counter while every sensor has a lane of
-one workgroup (256), in two launches beyond.  The maximum, minimum and sum of squares are
+one workgroup (256), in two launches beyond; with millions of sensors every step has a
+launch of its own.  The maximum, minimum and sum of squares are
 read and written again every step, so a step gathered twice, or not at all, shows.
 """
 import ctypes as C
@@ -33,12 +34,9 @@ def _plan(shape, nt):
     return DevicePlan([build_instance(kg, med, src, sen, pml_size=(3,) * len(shape), pml_alpha=(2.0,) * len(shape))])
 
 
-@pytest.mark.parametrize("shape", [(70, 66), (128, 64), (20, 18, 16), (32, 16, 24)])
-@pytest.mark.parametrize("sensors", [1, 255, 256, 257, 4500])
-def test_aggregates_follow_the_recorded_series(shape, sensors, monkeypatch):
+def _check(shape, sensors, nt, start, monkeypatch):
     from kwave_amd import _abi
 
-    nt, start = 30, 5
     idx = np.sort(np.random.default_rng(sensors).choice(int(np.prod(shape)), sensors, replace=False)).astype(np.int64)
 
     def records(steps):
@@ -62,3 +60,15 @@ def test_aggregates_follow_the_recorded_series(shape, sensors, monkeypatch):
         assert np.array_equal(agg[0], p.max(axis=0)) and np.array_equal(agg[1], p.min(axis=0))
         # nt - start squares and additions in FP32, each rounded by at most 2^-24 of the sum
         np.testing.assert_allclose(agg[2], (p.astype(np.float64) ** 2).sum(axis=0), rtol=2 * (nt - start) * 2.0 ** -24)
+
+
+@pytest.mark.parametrize("shape", [(70, 66), (128, 64), (20, 18, 16), (32, 16, 24)])
+@pytest.mark.parametrize("sensors", [1, 255, 256, 257, 4500])
+def test_aggregates_follow_the_recorded_series(shape, sensors, monkeypatch):
+    _check(shape, sensors, 30, 5, monkeypatch)
+
+
+@pytest.mark.parametrize("shape,sensors", [((160, 160, 120), 3000000), ((160, 160, 120), 3000001), ((150, 161, 125), 3018750)])
+def test_aggregates_of_very_many_sensors(shape, sensors, monkeypatch):
+    """Around the number from which every step of a block gathers in a kernel of its own."""
+    _check(shape, sensors, 14, 2, monkeypatch)
