@@ -13,7 +13,9 @@ namespace kw {
 // 128^2 (66 k lanes a group) 64.1 -> 59.9, 1024^2 power law 109.8 -> 103.1; beyond, the sixteen
 // scan lines of 256^2 to 640^2 lose (197.7 -> 201.6 at 150 k lanes, 218.5 at 300 k) and
 // 160^3 (512 k lanes an axis) 289 -> 324.  Plans of a batch share the chip with the others'
-// kernels and take half as many (small 3): the scan lines 176 -> 163 us a step.
+// kernels and take half as many (small 3): the scan lines 176 -> 163 us a step; eleven other
+// mixes (2 to 90 instances, 2 to 4 plans, 96^2 to 1024 x 768) differ less between the two limits
+// than between two runs.
 bool z_small(const Geom& g, int nb, int tpl, int groups) {
   if (g.small == 0) return false;
   return g.small == 2 || (int64_t)(g.rows / 2) * tpl * nb * groups <= (g.small == 3 ? 75000 : 150000);

@@ -41,7 +41,11 @@ constexpr int kGenMaxN = 4096;
 constexpr int kGenThreads = 256;
 constexpr int kGenMaxStages = 16;
 constexpr size_t kGenLds = 163840;     // LDS of a compute unit
-constexpr size_t kGenLdsShare = 32768;  // a workgroup's LDS where it can choose: several fit
+// A workgroup's LDS where it can choose.  us a step with 32 KB -> 64 KB: 330 x 333 x 310 4221 ->
+// 3708, 291 x 300 x 322 power law 5615 -> 5394, 200 x 180 x 170 and 108 x 90 x 75 with velocities
+// 1063 -> 964 and 190 -> 181; 400^3 6800 -> 6905, 150^3 power law 452 -> 471, 360 x 420 x 64
+// 966 -> 996; 2-D grids of 242 x 291 to 2000 x 1900 alike.  80 KB loses twice as much and gains less.
+constexpr size_t kGenLdsShare = 32768;
 
 struct GPlan {
   int n;

@@ -113,7 +113,7 @@ __device__ __forceinline__ void gather_point(const Geom& g, const Fields& fl, co
 // before, whose fields nothing changes before the next update.  A kernel of its own would
 // add its launch and one chain of latencies, 4 to 5 us, to every step (with the counter
 // advanced once a block as well, us per step: 128^2 30.0 -> 25.7, 512^2 power law 51.3 ->
-// 48.4, 64 maps of 128^2 58.5 -> 54.7).
+// 48.4, 64 maps of 128^2 58.5 -> 54.7).  Up to kGatherInPass sensors (kw_abi.hip).
 __device__ __forceinline__ void gather_blocks(const Geom& g, const Fields& fl, const Inst* inst, const ColArgs& a) {
   if (blockIdx.z) return;
   const int b = blockIdx.y;
@@ -322,7 +322,7 @@ __device__ __forceinline__ void set_lane(float2 (&a)[E], int m, int h, float v) 
 // registers, 2155 -> 2948 us; the momentum kernel forced from 3 to 4, 1904 -> 2808 us).
 //
 // What bounds the updates on large grids is memory (512^3: mass 1686 us = 4.5 TB/s of
-// its algorithmic bytes, eos 811 us = 4.6, momentum 1846 us = 4.4; a plain copy reaches
+// its algorithmic bytes, eos 811 us = 4.6, momentum 1750 us = 4.6; a plain copy reaches
 // 5.0), once their loads are issued in batches: element loops with a test inside (the
 // nonlinear flag, a source mode, a clamped row) had compiled into one block per element,
 // each load waited for alone.  Straight-line loops with the tests around them took the

@@ -569,7 +569,7 @@ def predict(model, cmaps, batch=512, features=False, tta=False, ranges=False):
     buffers and uploaded on a stream of its own, so that both copies of the next batch
     overlap the forward of the current one; the traces come back on a third stream, under
     the next forward, into a page-locked array that is returned as is (no further host
-    copy).  1024 maps, one stream -> three: 6.4 -> 4.6 ms."""
+    copy).  1024 maps, one stream -> three: 6.4-6.9 -> 4.5-5.3 ms (by machine)."""
     import torch
 
     dev = next(model.parameters()).device
